@@ -418,6 +418,36 @@ void res_table(const gra_cfg& c, std::vector<ResDev>& tab) {
   }
 }
 
+// Whether a run's screening nodes can take the point-folded FP64 form (gra_fold.h):
+// the continuum with one active trajectory and the power-law off-shell form factor (the
+// exponential ones fall so fast that loop and tree cancel to 1e-3 at some points, where
+// the two forms' rounding shows), and kinematics for which the form's series
+// hold to FP64 rounding anywhere in phase space: with E5, pT and k at their largest,
+// x = (m^2 + pT^2) / p+^2 bounds the relative change of p+ over the loop, and the series
+// of delta drops x^3 < 1e-17. A run at 13 TeV has x ~ 2e-7; runs beyond the bound
+// (beams below about 1.5 TeV, pairs at very large rapidity) keep the reference-order
+// nodes.
+bool fold_process(const gra_cfg& c, const RunParams& P) {
+  if (!c.screening || P.asym || P.regge_k < 0 || c.amp_precision != GRA_AMP_FP64) return false;
+  // the component form's rounding differs from node to node and averages over a loop:
+  // with a few nodes it stays at 3e-10 of the weight, and there is little to gain
+  if (P.n_fold < 64) return false;
+  if (c.process != GRA_PROC_REGGE_CON || c.w_central > 0.0 || c.offshellFF != 2) return false;
+  const double pT = c.fwd_pt_max, km = c.max_loop_kt;
+  const double y = std::max(std::fabs(c.rap_min), std::fabs(c.rap_max));
+  double E5;
+  if (c.phase_space == GRA_PS_F) {
+    E5 = std::hypot(P.f_Mmax, 2.0 * pT) * std::cosh(y);
+  } else {
+    const double kt = std::max(std::fabs(c.kt_min), std::fabs(c.kt_max));
+    E5 = 2.0 * std::hypot(c.m_central, 0.5 * kt + pT) * std::cosh(y);
+  }
+  if (!(E5 < 0.2 * P.sqrt_s)) return false;
+  const double b = 1.1 * c.m_beam * c.m_beam + (pT + km) * (pT + km);
+  const double pp = P.sqrt_s - 2.0 * E5 - std::sqrt(b);  // smallest p1+, p2-
+  return pp > 0.0 && b / (pp * pp) <= 2e-6;
+}
+
 void fill_params(const gra_cfg& c, RunParams& P) {
   std::memset(&P, 0, sizeof(P));
   P.process = c.process;
@@ -560,6 +590,13 @@ void fill_params(const gra_cfg& c, RunParams& P) {
   P.hfac = (c.loop_rule == GRA_LOOP_GAUSS) ? 1.0 : 9 * (P.step_phi * P.step_kt) / 64;
   P.nrm = 1.0 / (8.0 * (GRA_PI * GRA_PI) * P.s);
   P.kappa = P.nrm * P.hfac;
+  P.f_fsq = 1.0 / c.fc1 + 1.0 / c.fc2;
+  P.f_fpq = 1.0 / (c.fc1 * c.fc2);
+  P.f_ls0 = std::log2(c.regge_s0);
+  P.f_ibp = 1.0 / c.b_POW;
+  P.f_phr = P.ph_c / (2.0 * GRA_PI);
+  P.f_cb1 = P.pbeam1.e - P.pbeam1.z;
+  P.f_cb2 = P.pbeam2.e + P.pbeam2.z;
   // tensor pomeron
   P.tp_delta_P = c.tp_delta_P;
   P.tp_ap_P = c.tp_ap_P;
@@ -577,6 +614,10 @@ void fill_params(const gra_cfg& c, RunParams& P) {
   P.spin_frame = c.spin_frame;
   P.omega = c.regge_omega;
   P.m_rho = c.m_central;
+  // folded nodes: the Simpson rows phi = 0 and 2 pi are one direction, the Gauss
+  // rule's azimuths are distinct
+  P.n_fold = (c.loop_rule == GRA_LOOP_GAUSS ? c.n_loop_phi + 1 : c.n_loop_phi) * (c.n_loop_kt + 1);
+  P.fold = fold_process(c, P) ? 1 : 0;
 }
 
 // One eikonal table through the cache directory dir (none: nullptr), as
@@ -758,10 +799,22 @@ int build_eikonal(gra_handle* h, const char* cache_dir) {
   }
   const size_t b0 = sizeof(NodeConst) * NN, b1 = sizeof(NodeF32) * NN,
                b2 = sizeof(NodeRow) * rows.size();
-  if (h->d_nodes.ensure(b0 + b1 + b2)) return fail(h, GRA_E_NOMEM, "node table");
+  // the folded nodes: entries of rows that coincide (phi = 0 and 2 pi) added
+  const size_t b3 = fold_node_offset(P), n_fold = (size_t)P.n_fold;
+  std::vector<NodeFold> nf(n_fold);
+  for (size_t k = 0; k < NN; ++k) {
+    const NodeConst& nd = h->nodes[k];
+    NodeFold& f = nf[k % n_fold];
+    if (k < n_fold) f = {nd.kx, nd.ky, 0.0, 0.0};
+    f.cre += nd.w * nd.kt * nd.aeik_re;
+    f.cim += nd.w * nd.kt * nd.aeik_im;
+  }
+  if (h->d_nodes.ensure(b3 + sizeof(NodeFold) * n_fold)) return fail(h, GRA_E_NOMEM, "node table");
   GRA_HIP_CHECK(h, hipMemcpy(h->d_nodes.p, h->nodes.data(), b0, hipMemcpyHostToDevice));
   GRA_HIP_CHECK(h, hipMemcpy((char*)h->d_nodes.p + b0, n32.data(), b1, hipMemcpyHostToDevice));
   GRA_HIP_CHECK(h, hipMemcpy((char*)h->d_nodes.p + b0 + b1, rows.data(), b2, hipMemcpyHostToDevice));
+  GRA_HIP_CHECK(h, hipMemcpy((char*)h->d_nodes.p + b3, nf.data(), sizeof(NodeFold) * n_fold,
+                             hipMemcpyHostToDevice));
   return GRA_OK;
 }
 

@@ -9,6 +9,13 @@
 
 namespace gra_hip {
 
+// Device node table: one NodeConst per loop node, the NodeF32 entries, one NodeRow per
+// phi row, and from fold_node_offset on the P.n_fold NodeFold entries
+inline size_t fold_node_offset(const RunParams& P) {
+  const size_t rows = (size_t)P.nphi + 1, nn = rows * (P.nkt + 1);
+  return (sizeof(NodeConst) * nn + sizeof(NodeF32) * nn + sizeof(NodeRow) * rows + 15) / 16 * 16;
+}
+
 #define GRA_DECLARE_INTEGRAND_LAUNCHERS(NS)                                                        \
   namespace NS {                                                                                   \
   size_t loop_record_bytes(const RunParams& P);                                                    \

@@ -77,6 +77,13 @@ struct RunParams {
   int32_t tp_mode, pad_tp;
   double tp_delta_P, tp_ap_P, tp_gPNN, tp_gPvv0, tp_gPvv1, tp_mp_ff, m_rho;
   double tp_gP;  // Pomeron-pseudoscalar-pseudoscalar coupling of the 2xS mode
+  // FP64 screening nodes in point-folded form (gra_fold.h): on, number of nodes, and
+  // the amplitude's constants in base 2
+  int32_t fold, n_fold;
+  double f_fsq, f_fpq;    // (1 - t / fc1)(1 - t / fc2) = 1 - fsq t + fpq t^2
+  double f_ls0, f_ibp;    // log2 s0, 1 / b_POW
+  double f_phr;           // ph_c / (2 pi)
+  double f_cb1, f_cb2;    // E - |p_z| of the beams from their rounded components
   // resonances (PP[RES+CON]): device table of nres entries
   const ResDev* res;
   int32_t nres, spin_gen, spin_dec, spin_frame;
@@ -103,4 +110,9 @@ struct NodeF32 {
 };
 struct NodeRow {
   float c, s;  // cos(phi_i), sin(phi_i)
+};
+// Node of the point-folded FP64 loop: k and the node's factor w kt A_eik. The rows
+// phi = 0 and 2 pi of the Simpson grid are one direction and share their entries.
+struct NodeFold {
+  double kx, ky, cre, cim;
 };
