@@ -418,6 +418,63 @@ void res_table(const gra_cfg& c, std::vector<ResDev>& tab) {
   }
 }
 
+// Coefficients of a diagonal density's spin traces (trace1, trace2 in gra_fold_res.h):
+// |d^1_{+-1,+-1}|^2 summed and |d^1_{.0}|^2; |d^2_{0,+-2}|^2 = 3/8 sin^4,
+// |d^2_{0,+-1}|^2 = 3/2 sin^2 cos^2, d^2_{00} = (3 cos^2 - 1) / 2
+void spin1_coefs(const ResDev& R, double* c) {
+  c[0] = R.rho_re[0] + R.rho_re[8];
+  c[1] = R.rho_re[4];
+}
+void spin2_coefs(const ResDev& R, double* c) {
+  c[0] = 0.375 * (R.rho_re[0] + R.rho_re[24]);
+  c[1] = 1.5 * (R.rho_re[6] + R.rho_re[18]);
+  c[2] = R.rho_re[12];
+}
+bool diagonal_density(const gra_res& q) {
+  const int n = 2 * q.J + 1;
+  for (int a = 0; a < n; ++a)
+    for (int b = 0; b < n; ++b)
+      if (a != b && (q.rho_re[a * n + b] != 0.0 || q.rho_im[a * n + b] != 0.0)) return false;
+  return true;
+}
+// Resonances with equal spin densities share one entry and one trace per node
+void fold_res_table(const gra_cfg& c, const std::vector<ResDev>& tab, FoldResTab& T) {
+  std::memset(&T, 0, sizeof(T));
+  int nc[3] = {0, 0, 0};
+  int first[3][GRA_MAX_RES];
+  const int n = (int)tab.size();
+  for (int r = 0; r < n; ++r) {
+    const ResDev& R = tab[r];
+    if (R.J == 0) continue;
+    int k = 0;
+    while (k < nc[R.J] && (std::memcmp(tab[first[R.J][k]].rho_re, R.rho_re, sizeof(R.rho_re)) ||
+                           std::memcmp(tab[first[R.J][k]].rho_im, R.rho_im, sizeof(R.rho_im))))
+      ++k;
+    if (k == nc[R.J]) {
+      first[R.J][nc[R.J]++] = r;
+      if (R.J == 1) spin1_coefs(R, T.c1[k]);
+      else spin2_coefs(R, T.c2[k]);
+    }
+    T.cls[r] = k;
+  }
+  int sum_of[GRA_MAX_RES];
+  for (int k = 0; k < GRA_MAX_RES; ++k) sum_of[k] = -1;
+  for (int r = 0; r < n; ++r)
+    if (tab[r].J == 2 && c.spin_gen && sum_of[T.cls[r]] < 0) {
+      T.prod2[T.n2] = T.cls[r];
+      sum_of[T.cls[r]] = 1 + T.n2++;
+    }
+  for (int r = 0; r < n; ++r) {
+    if (tab[r].photo) {
+      T.ph_cls[T.nph] = c.spin_gen ? T.cls[r] : -1;
+      T.beta[T.nph] = 0.5 * tab[r].B0 * 1.4426950408889634;
+      T.slot[r] = 1 + T.n2 + T.nph++;
+    } else {
+      T.slot[r] = (tab[r].J == 2 && c.spin_gen) ? sum_of[T.cls[r]] : 0;
+    }
+  }
+}
+
 // Whether a run's screening nodes can take the point-folded FP64 form (gra_fold.h):
 // the continuum with one active trajectory and the power-law off-shell form factor (the
 // exponential ones fall so fast that loop and tree cancel to 1e-3 at some points, where
@@ -432,7 +489,14 @@ bool fold_process(const gra_cfg& c, const RunParams& P) {
   // the component form's rounding differs from node to node and averages over a loop:
   // with a few nodes it stays at 3e-10 of the weight, and there is little to gain
   if (P.n_fold < 64) return false;
-  if (c.process != GRA_PROC_REGGE_CON || c.w_central > 0.0 || c.offshellFF != 2) return false;
+  if (c.process == GRA_PROC_TENSOR_CON || c.w_central > 0.0 || c.offshellFF != 2) return false;
+  if (c.process != GRA_PROC_REGGE_CON) {
+    // resonances: the Gottfried-Jackson axis moves with the node, the photon terms take
+    // trajectory 0, and the traces are those of diagonal densities
+    if (c.spin_frame == GRA_FRAME_GJ) return false;
+    for (int r = 0; r < c.n_res; ++r)
+      if ((c.res[r].J == 1 && P.regge_k != 0) || !diagonal_density(c.res[r])) return false;
+  }
   const double pT = c.fwd_pt_max, km = c.max_loop_kt;
   const double y = std::max(std::fabs(c.rap_min), std::fabs(c.rap_max));
   double E5;
@@ -597,6 +661,9 @@ void fill_params(const gra_cfg& c, RunParams& P) {
   P.f_phr = P.ph_c / (2.0 * GRA_PI);
   P.f_cb1 = P.pbeam1.e - P.pbeam1.z;
   P.f_cb2 = P.pbeam2.e + P.pbeam2.z;
+  P.f_ibz = 1.0 / P.pbeam1.z;
+  P.f_i4mp2 = 0.25 / (c.tp_mp_ff * c.tp_mp_ff);
+  P.fres = nullptr;
   // tensor pomeron
   P.tp_delta_P = c.tp_delta_P;
   P.tp_ap_P = c.tp_ap_P;
@@ -799,16 +866,19 @@ int build_eikonal(gra_handle* h, const char* cache_dir) {
   }
   const size_t b0 = sizeof(NodeConst) * NN, b1 = sizeof(NodeF32) * NN,
                b2 = sizeof(NodeRow) * rows.size();
-  // the folded nodes: entries of rows that coincide (phi = 0 and 2 pi) added
-  const size_t b3 = fold_node_offset(P), n_fold = (size_t)P.n_fold;
+  // the folded nodes, kt by kt; rows that coincide (phi = 0 and 2 pi) are added
+  const size_t b3 = fold_node_offset(P), n_fold = (size_t)P.n_fold, n_row = n_fold / (NK + 1);
   std::vector<NodeFold> nf(n_fold);
-  for (size_t k = 0; k < NN; ++k) {
-    const NodeConst& nd = h->nodes[k];
-    NodeFold& f = nf[k % n_fold];
-    if (k < n_fold) f = {nd.kx, nd.ky, 0.0, 0.0};
-    f.cre += nd.w * nd.kt * nd.aeik_re;
-    f.cim += nd.w * nd.kt * nd.aeik_im;
-  }
+  h->P.n_fold_ref = 0;
+  for (int i = 0; i <= NP; ++i)
+    for (int j = 0; j <= NK; ++j) {
+      const NodeConst& nd = h->nodes[(size_t)i * (NK + 1) + j];
+      NodeFold& f = nf[j * n_row + i % n_row];
+      if ((size_t)i < n_row) f = {nd.kx, nd.ky, 0.0, 0.0};
+      f.cre += nd.w * nd.kt * nd.aeik_re;
+      f.cim += nd.w * nd.kt * nd.aeik_im;
+      if ((size_t)i < n_row && nd.kt < kFoldRefKt) ++h->P.n_fold_ref;
+    }
   if (h->d_nodes.ensure(b3 + sizeof(NodeFold) * n_fold)) return fail(h, GRA_E_NOMEM, "node table");
   GRA_HIP_CHECK(h, hipMemcpy(h->d_nodes.p, h->nodes.data(), b0, hipMemcpyHostToDevice));
   GRA_HIP_CHECK(h, hipMemcpy((char*)h->d_nodes.p + b0, n32.data(), b1, hipMemcpyHostToDevice));
@@ -1036,13 +1106,17 @@ int create_handle(const gra_cfg* cfg, const char* eikonal_dir, gra_handle** out)
   if (h->P.nres > 0) {
     std::vector<ResDev> tab;
     res_table(h->cfg, tab);
+    FoldResTab ft;
+    fold_res_table(h->cfg, tab, ft);
     const size_t b = sizeof(ResDev) * tab.size();
-    if (h->d_res.ensure(b) ||
-        hipMemcpy(h->d_res.p, tab.data(), b, hipMemcpyHostToDevice) != hipSuccess) {
+    if (h->d_res.ensure(b + sizeof(ft)) ||
+        hipMemcpy(h->d_res.p, tab.data(), b, hipMemcpyHostToDevice) != hipSuccess ||
+        hipMemcpy((char*)h->d_res.p + b, &ft, sizeof(ft), hipMemcpyHostToDevice) != hipSuccess) {
       gra_hip_destroy(h);
       return set_global_error(GRA_E_HIP, "gra_hip_create: resonance table upload failed");
     }
     h->P.res = (const ResDev*)h->d_res.p;
+    h->P.fres = (const FoldResTab*)((const char*)h->d_res.p + b);
   }
   if (h->cfg.screening) {
     const int r = build_eikonal(h, eikonal_dir);

@@ -209,6 +209,7 @@ __device__ __forceinline__ void fold_point(const RunParams& P, const FoldRec& r,
 struct FoldKin {
   double del1, del2, a5, a6;
   double t1, t2, s13, s24, s14, s23, th, tu;
+  double dz, dq;  // of q1 = p_a - p1: z component, and z component + d_a - energy
 };
 __device__ __forceinline__ void fold_kin(const RunParams& P, const FoldPt& F, double kx, double ky,
                                          FoldKin& K) {
@@ -235,31 +236,33 @@ __device__ __forceinline__ void fold_kin(const RunParams& P, const FoldPt& F, do
   K.s24 = F.S24 - L4;
   K.th = K.t1 + (F.T3 + L3);
   K.tu = K.t1 + (F.T4 + L4);
+  K.dz = 0.5 * ((F.w1 + K.del1) + (K.del2 - P.f_cb1));
+  K.dq = K.del1;
 }
 
-// The closed form of SolvePz sums ~30 terms of order s^2; its p1z carries a rounding
-// offset that is largely common to the nodes of a point (0.6e-12 GeV, and 0.7e-12 GeV
-// from node to node). It reaches t^ and u^ at the 1e-11 level of the amplitude, which
-// a screened weight that nearly cancels against its tree amplitude amplifies: the
-// offset is sampled at a few nodes and kept, so that loop and tree amplitude see the
-// same one. Returns p1z(closed form) - p1z at the node.
-__device__ __forceinline__ double fold_offset(const RunParams& P, const FoldRec& r,
-                                              const FoldPt& F, double kx, double ky) {
-  FoldKin K;
-  fold_kin(P, F, kx, ky, K);
-  const double ax = r.p1x - kx, ay = r.p1y - ky, bx = r.p2x + kx, by = r.p2y + ky;
-  const double z = solvepz(r.m1, r.m2, msq(ax * ax + ay * ay), msq(bx * bx + by * by),
-                           r.dt[0].z + r.dt[1].z, r.dt[0].e + r.dt[1].e, P);
-  // p_beam,z - p1z = (X+ + delta1 + delta2) / 2 - d_a
-  return (z - P.pbeam1.z) + 0.5 * ((F.w1 + K.del1) + (K.del2 - P.f_cb1));
-}
-// Moves p1z and |p2z| of every node by the offset
-__device__ __forceinline__ void fold_shift(double off, FoldPt& F) {
-  const double d = 2.0 * off;  // of p1+ and p2-
-  F.w1 -= d;
-  F.w2 -= d;
-  F.T3 = __builtin_fma(d, F.p3m, F.T3);
-  F.T4 = __builtin_fma(d, F.p4m, F.T4);
+// t1, t2, t^, u^ and q1 of a node from the momentum components, in the reference's operation
+// order. The component form rounds them at the 1e-12 GeV^2 level (E eps times an energy
+// transfer), the tree amplitude with them, and a screened weight that nearly cancels
+// against its tree amplitude shows it at 1e-10. Only nodes near the tree point matter:
+// the loop's weight sits at small k, and further out the roundings differ from node to
+// node and average. So the nodes below kFoldRefKt (13% of the Simpson grid), which
+// come first in the node table, take this form and weights keep the reference's rounding
+// to 3e-11; the others take it at 1e-10.
+__device__ __forceinline__ void fold_kin_components(const RunParams& P, const FoldRec& r,
+                                                    double kx, double ky, FoldKin& K) {
+  const double p1x = r.p1x - kx, p1y = r.p1y - ky, p2x = r.p2x + kx, p2y = r.p2y + ky;
+  const double pt1 = msq(p1x * p1x + p1y * p1y), pt2 = msq(p2x * p2x + p2y * p2y);
+  const dv4 X = v4add(r.dt[0], r.dt[1]);
+  const double p1z = solvepz(r.m1, r.m2, pt1, pt2, X.z, X.e, P);
+  const double p2z = -(X.z + p1z);
+  const dv4 q1 = v4sub(P.pbeam1, v4m(p1x, p1y, p1z, msq(r.m1 * r.m1 + pt1 * pt1 + p1z * p1z)));
+  const dv4 q2 = v4sub(P.pbeam2, v4m(p2x, p2y, p2z, msq(r.m2 * r.m2 + pt2 * pt2 + p2z * p2z)));
+  K.t1 = m2of(q1);
+  K.t2 = m2of(q2);
+  K.th = m2of(v4sub(q1, r.dt[0])) - P.m_prop2;
+  K.tu = m2of(v4sub(q1, r.dt[1])) - P.m_prop2;
+  K.dz = q1.z;
+  K.dq = (q1.z + P.f_cb1) - q1.e;
 }
 
 // (1 - t / fc1)(1 - t / fc2), the inverse of form::S3F

@@ -29,6 +29,21 @@ struct ResDev {
 constexpr int32_t kTp2xV = 0;  // vector-meson pair
 constexpr int32_t kTp2xS = 1;  // pseudoscalar pair
 
+constexpr double kFoldRefKt = 0.4;  // GeV, see fold_kin_components (gra_fold.h)
+
+// Resonances of the point-folded FP64 nodes (gra_fold_res.h). A point keeps 1 + n2 + nph
+// complex coefficient sums: the one without a production trace, one for each J = 2 spin
+// density, one for each photoproduced resonance.
+struct FoldResTab {
+  int32_t n2, nph;
+  int32_t cls[GRA_MAX_RES];     // spin density of resonance r (J > 0) among c1 (J = 1) or c2
+  int32_t slot[GRA_MAX_RES];    // the sum that resonance r joins
+  int32_t prod2[GRA_MAX_RES];   // spin density of sum 1 + c
+  int32_t ph_cls[GRA_MAX_RES];  // spin density of photoproduced resonance k, -1: no trace
+  double beta[GRA_MAX_RES];     // its slope B0 log2(e) / 2
+  double c1[GRA_MAX_RES][2], c2[GRA_MAX_RES][3];  // trace1, trace2
+};
+
 struct RunParams {
   int32_t process, amp_mode, dim, screening;
   // beams and invariants
@@ -77,13 +92,15 @@ struct RunParams {
   int32_t tp_mode, pad_tp;
   double tp_delta_P, tp_ap_P, tp_gPNN, tp_gPvv0, tp_gPvv1, tp_mp_ff, m_rho;
   double tp_gP;  // Pomeron-pseudoscalar-pseudoscalar coupling of the 2xS mode
-  // FP64 screening nodes in point-folded form (gra_fold.h): on, number of nodes, and
-  // the amplitude's constants in base 2
-  int32_t fold, n_fold;
+  // FP64 screening nodes in point-folded form (gra_fold.h): on, number of nodes, of them
+  // with t from components, and the amplitude's constants in base 2
+  int32_t fold, n_fold, n_fold_ref, pad_fold;
   double f_fsq, f_fpq;    // (1 - t / fc1)(1 - t / fc2) = 1 - fsq t + fpq t^2
   double f_ls0, f_ibp;    // log2 s0, 1 / b_POW
   double f_phr;           // ph_c / (2 pi)
   double f_cb1, f_cb2;    // E - |p_z| of the beams from their rounded components
+  double f_ibz, f_i4mp2;  // 1 / p_z of beam 1, 1 / (2 m_p)^2 of the photon flux
+  const FoldResTab* fres;
   // resonances (PP[RES+CON]): device table of nres entries
   const ResDev* res;
   int32_t nres, spin_gen, spin_dec, spin_frame;
@@ -111,8 +128,9 @@ struct NodeF32 {
 struct NodeRow {
   float c, s;  // cos(phi_i), sin(phi_i)
 };
-// Node of the point-folded FP64 loop: k and the node's factor w kt A_eik. The rows
-// phi = 0 and 2 pi of the Simpson grid are one direction and share their entries.
+// Node of the point-folded FP64 loop: k and the node's factor w kt A_eik, in order of
+// kt. The rows phi = 0 and 2 pi of the Simpson grid are one direction and share their
+// entries.
 struct NodeFold {
   double kx, ky, cre, cim;
 };

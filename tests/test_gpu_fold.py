@@ -1,8 +1,9 @@
-"""The point-folded FP64 screening nodes (gra_fold.h) against the oracle's
+"""The point-folded FP64 screening nodes (gra_fold.h, gra_fold_res.h) against the oracle's
 reference-order loop, over what the dispatch sends there: both phase-space classes,
 every off-shell form factor, both loop rules down to a single node, launches that do
-not fill a wave or a block, and beams below the form's range (which keep the
-reference-order nodes).
+not fill a wave or a block, the resonances' frames, spin switches and densities, and
+runs outside the form's range (low beams, few nodes, other form factors, the
+Gottfried-Jackson frame), which keep the reference-order nodes.
 
 Tolerance. Folded and reference-order nodes differ by the rounding of the component
 form: t1, t2, t^ and u^ carry about 1e-12 GeV^2 of noise from node to node (E eps
@@ -40,13 +41,61 @@ CASES = {
 }
 
 
-@pytest.mark.parametrize("name", sorted(CASES))
+def mixed_density(cfg):
+    """Full complex spin densities, a different one for each resonance with J > 0."""
+    rng = np.random.default_rng(5)
+    for r in range(cfg.n_res):
+        q = cfg.res[r]
+        m = 2 * q.J + 1
+        a = rng.normal(size=(m, m)) + 1j * rng.normal(size=(m, m))
+        rho = a @ a.conj().T
+        rho /= np.trace(rho).real
+        for k, v in enumerate(rho.reshape(-1)):
+            q.rho_re[k], q.rho_im[k] = v.real, v.imag
+
+
+def one_photoproduced(cfg):
+    """The rho(770) alone, beside the continuum."""
+    cfg.res[0] = cfg.res[7]
+    cfg.n_res = 1
+
+
+def all_tensors(cfg):
+    """Eight J = 2 resonances, each with its own density: the most sums a point can have."""
+    for r in range(8):
+        mass, width = cfg.res[r].mass, cfg.res[r].width
+        cfg.res[r] = cfg.res[4]
+        cfg.res[r].mass, cfg.res[r].width = mass, width
+    mixed_density(cfg)
+
+
+RES_CASES = {
+    "res_collins_soper": ({}, None),
+    "res_helicity": ({"spin_frame": abi.GRA_FRAME_HX}, None),
+    "res_cm": ({"spin_frame": abi.GRA_FRAME_CM}, None),
+    "res_no_production_spin": ({"spin_gen": 0}, None),
+    "res_no_decay_spin": ({"spin_dec": 0}, None),
+    "res_full_densities": ({}, mixed_density),
+    "res_one_photoproduced": ({}, one_photoproduced),
+    "res_all_tensors": ({}, all_tensors),
+    "res_no_continuum": ({"process": abi.GRA_PROC_RES}, None),
+    "res_none": ({"n_res": 0}, None),
+}
+
+
+@pytest.mark.parametrize("name", sorted(CASES) + sorted(RES_CASES))
 def test_folded_nodes(name):
-    preset, n, over = CASES[name]
+    change = None
+    if name in CASES:
+        preset, n, over = CASES[name]
+    else:
+        preset, n, (over, change) = 7, 65, RES_CASES[name]
     cfg = small_tables(abi.cfg_default(preset), 500)
     cfg.amp_precision = abi.GRA_AMP_FP64
     for key, value in over.items():
         setattr(cfg, key, value)
+    if change:
+        change(cfg)
     print(f"case: {name}, {n} points", flush=True)
     u = np.random.default_rng(71).random((n, cfg.dim))
     with MContinuum(cfg) as P:
