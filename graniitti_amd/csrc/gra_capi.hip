@@ -456,6 +456,8 @@ void fold_res_table(const gra_cfg& c, const std::vector<ResDev>& tab, FoldResTab
       else spin2_coefs(R, T.c2[k]);
     }
     T.cls[r] = k;
+    for (int a = 0; a < 2 * R.J + 1; ++a)
+      if (R.rho_re[a * (2 * R.J + 2)] != 0.0) (R.J == 1 ? T.mask1 : T.mask2) |= 1 << a;
   }
   int sum_of[GRA_MAX_RES];
   for (int k = 0; k < GRA_MAX_RES; ++k) sum_of[k] = -1;
@@ -485,7 +487,9 @@ void fold_res_table(const gra_cfg& c, const std::vector<ResDev>& tab, FoldResTab
 // (beams below about 1.5 TeV, pairs at very large rapidity) keep the reference-order
 // nodes.
 bool fold_process(const gra_cfg& c, const RunParams& P) {
-  if (!c.screening || P.asym || P.regge_k < 0 || c.amp_precision != GRA_AMP_FP64) return false;
+  if (!c.screening || P.asym || P.regge_k < 0) return false;
+  // the FP32 continuum has a node of its own
+  if (c.process == GRA_PROC_REGGE_CON && c.amp_precision != GRA_AMP_FP64) return false;
   // the component form's rounding differs from node to node and averages over a loop:
   // with a few nodes it stays at 3e-10 of the weight, and there is little to gain
   if (P.n_fold < 64) return false;

@@ -207,3 +207,172 @@ __device__ __forceinline__ cxd fold_photo_node(const RunParams& P, const FoldRes
   }
   return A;
 }
+
+// ---------------------------------------------------------------------------
+// The FP32-amplitude form (res_sum32 and regge_me4_32, gra_res.h) on folded kinematics:
+// the same FP32 operations on the same FP64 scalars, with what the node does not change
+// taken out of the loop. Per resonance and point: Breit-Wigner, form factor and decay
+// amplitude (FoldRes32, formed by the resonance's lane); per node and spin: the rows
+// g_a of the production trace, shared by the resonances of that spin; of the trace only
+// the density's diagonal (fold_process), whose other terms add exact zeros.
+// ---------------------------------------------------------------------------
+struct FoldRes32 {
+  cxf bw;     // times rff for a photoproduced resonance
+  cxf decay;  // times the production coupling where there is no production trace
+  float rff;
+};
+__device__ __forceinline__ FoldRes32 fold_res32_coef(const RunParams& P, int r, float m2, float mA,
+                                                     float mB, float thd, float phd,
+                                                     const RotD32& D) {
+#pragma clang fp contract(fast)
+  const ResDev& R = P.res[r];
+  FoldRes32 z;
+  z.bw = cbw32(R, m2, mA, mB);
+  const float dm = m2 - (float)R.M02;
+  z.rff = __expf(-(dm * dm) / (float)R.gFF4);
+  z.decay = decay_amp32(P, R, thd, phd, D);
+  if (R.photo) z.bw = rf_scale(z.bw, z.rff);
+  if (!P.spin_gen || R.J == 0) z.decay = cfmul(cf((float)R.g_re, (float)R.g_im), z.decay);
+  return z;
+}
+
+// g_a of the rows lambda_r (spin_trace32) for the diagonal entries a in mask
+template <int J, int NROW>
+__device__ __forceinline__ void fold_rows32(const int* lam, const float* T, float c, float s,
+                                            float cd_, float sd, const RotD32& D, int mask,
+                                            float* nrm) {
+#pragma clang fp contract(fast)
+  constexpr int n = 2 * J + 1;
+  cxf ph_[n];
+  ph_[J] = cf(1.f, 0.f);
+#pragma unroll
+  for (int k = 1; k <= J; ++k) {
+    ph_[J + k] = cfmul(ph_[J + k - 1], cf(cd_, sd));
+    ph_[J - k] = cf(ph_[J + k].re, -ph_[J + k].im);
+  }
+#pragma unroll
+  for (int r = 0; r < NROW; ++r) {
+    cxf f[n];
+#pragma unroll
+    for (int j = 0; j < n; ++j) f[j] = rf_scale(ph_[j], T[r] * wigner_d32(c, s, lam[r], j - J, J));
+#pragma unroll
+    for (int a = 0; a < n; ++a) {
+      nrm[r * n + a] = 0.f;
+      if (!(mask & (1 << a))) continue;  // wave-uniform
+      cxf acc = cf(0.f, 0.f);
+#pragma unroll
+      for (int j = 0; j < n; ++j)
+        acc = rf_add(acc, rf_scale(f[j], J == 1 ? D.d1[a][j] : D.d2[a][j]));
+      nrm[r * n + a] = cfmul(acc, cf(acc.re, -acc.im)).re;
+    }
+  }
+}
+// The trace's terms in spin_trace32's order
+template <int J, int NROW>
+__device__ __forceinline__ float fold_trace32(const ResDev& R, const float* nrm) {
+  constexpr int n = 2 * J + 1;
+  float tr = 0.f;
+#pragma unroll
+  for (int r = 0; r < NROW; ++r)
+#pragma unroll
+    for (int a = 0; a < n; ++a) {
+      const float term = (float)R.rho_re[a * n + a] * nrm[r * n + a];
+      tr = tr + term;
+    }
+  return tr;
+}
+
+struct FoldRes32Pt {
+  float m2, V;   // m_X^2 and its flux factor
+  RotD32 D;
+};
+// MRegge::PhotoProp without its slope factor: eta e^{i ph t} and s^alpha
+__device__ __forceinline__ cxf photo_eta32(const RunParams& P, float s, float t, float& pw) {
+#pragma clang fp contract(fast)
+  const float alpha = (float)P.regge_a0[0] + (float)P.regge_ap[0] * t;
+  float sn, cs;
+  __sincosf((float)((-GRA_PI / 2.0) * P.regge_ap[0]) * t, &sn, &cs);
+  pw = rf_pow(s, alpha);
+  return cfmul(cf((float)P.eta0_re[0], (float)P.eta0_im[0]), cf(cs, sn));
+}
+
+// The amplitude at a node: regge_me4_32 + res_sum32
+__device__ __forceinline__ cxf fold_node32(const RunParams& P, const FoldResTab& T,
+                                           const FoldRes32Pt& R32, const FoldRes32* coef, int st,
+                                           const FoldKin& K, double s1d, double s2d, double dz2,
+                                           dv4 q1b) {
+#pragma clang fp contract(fast)
+  const float s1 = (float)s1d, s2 = (float)s2d;
+  const float t1 = (float)K.t1, t2 = (float)K.t2;
+  const float FF_A = (float)P.gN_P * s3f32(P, t1), FF_B = (float)P.gN_P * s3f32(P, t2);
+  const cxf pr12 = cfmul(regge_prop32(P, s1, t1), regge_prop32(P, s2, t2));
+  const float cont = 2.f * FF_A * FF_B * R32.V;
+  float n1[9], n2[5];
+  if (P.spin_gen) {
+    float thq, phq, s, c, sd, cd_;
+    theta_phi32(q1b, thq, phq);
+    __sincosf(0.5f * thq, &s, &c);
+    __sincosf(phq - R32.D.phR, &sd, &cd_);
+    if (T.mask1) {
+      const int lam[3] = {1, 0, -1};
+      const float T1[3] = {-0.697f, -0.169f, 0.697f};
+      fold_rows32<1, 3>(lam, T1, c, s, cd_, sd, R32.D, T.mask1, n1);
+    }
+    if (T.mask2) {
+      const int lam[1] = {0};
+      const float T2[1] = {1.f};
+      fold_rows32<2, 1>(lam, T2, c, s, cd_, sd, R32.D, T.mask2, n2);
+    }
+  }
+  float gf1 = 0.f, gf2 = 0.f, pw1 = 0.f, pw2 = 0.f;
+  cxf eta1 = cf(0.f, 0.f), eta2 = eta1;
+  if (T.nph > 0) {
+    const float x1 = (float)(K.dz * P.f_ibz), x2 = (float)(dz2 * P.f_ibz), mp = (float)P.tp_mp_ff;
+    gf1 = sqrtf(fmaxf(coh_flux32(x1, t1, (float)sqrt_pos64(K.a5), mp) / x1, 0.f));
+    gf2 = sqrtf(fmaxf(coh_flux32(x2, t2, (float)sqrt_pos64(K.a6), mp) / x2, 0.f));
+    eta1 = photo_eta32(P, s1, t1, pw1);
+    eta2 = photo_eta32(P, s2, t2, pw2);
+  }
+  cxf A = cf(0.f, 0.f);
+  int c1 = -1, c2 = -1;  // the densities that sc1, sc2 = sqrt(2J + 1) sqrt(trace) belong to
+  float sc1 = 0.f, sc2 = 0.f;
+  for (int r = 0; r < P.nres; ++r) {
+    const ResDev& R = P.res[r];
+    const FoldRes32 z = coef[r * st];
+    cxf spin = z.decay;
+    if (P.spin_gen && R.J != 0) {
+      const int c = T.cls[r];
+      if (R.J == 1 && c != c1) {
+        c1 = c;
+        sc1 = sqrtf(2.f * R.J + 1.f) * sqrtf(fmaxf(fold_trace32<1, 3>(R, n1), 0.f));
+      } else if (R.J == 2 && c != c2) {
+        c2 = c;
+        sc2 = sqrtf(2.f * R.J + 1.f) * sqrtf(fmaxf(fold_trace32<2, 1>(R, n2), 0.f));
+      }
+      spin = cfmul(rf_scale(cf((float)R.g_re, (float)R.g_im), R.J == 1 ? sc1 : sc2), z.decay);
+    }
+    if (R.photo) {
+      const float B0 = (float)R.B0;
+      const float F1 = (float)P.gN_P * __expf(0.5f * B0 * t1);
+      const float F2 = (float)P.gN_P * __expf(0.5f * B0 * t2);
+      const cxf A12 = rf_add(rf_scale(cfmul(z.bw, rf_scale(eta1, pw1 * F1)), gf2),
+                             rf_scale(cfmul(z.bw, rf_scale(eta2, pw2 * F2)), gf1));
+      A = rf_add(A, cfmul(A12, spin));
+    } else {
+      A = rf_add(A, rf_scale(cfmul(cfmul(pr12, z.bw), spin), cont * z.rff));
+    }
+  }
+  if (P.process != GRA_PROC_RES) {
+    Kin k;
+    k.t1 = K.t1;
+    k.t2 = K.t2;
+    k.ss13 = K.s13;
+    k.ss24 = K.s24;
+    k.ss14 = K.s14;
+    k.ss23 = K.s23;
+    k.t_hat = K.th + P.m_prop2;
+    k.u_hat = K.tu + P.m_prop2;
+    A = rf_add(A, regge_me4_32(P, k));
+  }
+  return A;
+}

@@ -36,6 +36,7 @@ constexpr double kFoldRefKt = 0.4;  // GeV, see fold_kin_components (gra_fold.h)
 // density, one for each photoproduced resonance.
 struct FoldResTab {
   int32_t n2, nph;
+  int32_t mask1, mask2;         // diagonal entries that a J = 1 (J = 2) density has, as bits
   int32_t cls[GRA_MAX_RES];     // spin density of resonance r (J > 0) among c1 (J = 1) or c2
   int32_t slot[GRA_MAX_RES];    // the sum that resonance r joins
   int32_t prod2[GRA_MAX_RES];   // spin density of sum 1 + c

@@ -441,7 +441,10 @@ __device__ __forceinline__ cxf cbw32(const ResDev& R, float m2, float mA, float 
     if (R.J == 1) num = -(1.f - r);
     if (R.J == 2) num = -(7.f / 6.f - (4.f / 3.f) * r + (2.f / 3.f) * (r * r));
   }
-  const float iden = __builtin_amdgcn_rcpf(a * a + b * b);
+  // sums of two products are fused explicitly here and in coh_flux32: which product the
+  // compiler would fuse depends on the code around, and the two nodes that use these
+  // functions (general and point-folded) have to round alike
+  const float iden = __builtin_amdgcn_rcpf(fmaf(b, b, a * a));
   return cf(num * a * iden, -num * b * iden);
 }
 __device__ __forceinline__ float coh_flux32(float xi, float t, float pt, float mp) {
@@ -451,10 +454,10 @@ __device__ __forceinline__ float coh_flux32(float xi, float t, float pt, float m
   const float GE = (1.f - 0.24f * tau) / (1.f + tau * (10.98f + tau * (12.82f + 21.97f * tau)));
   const float GM = 2.792847337f * ((1.f + 0.12f * tau) /
                                    (1.f + tau * (10.97f + tau * (18.86f + 6.55f * tau))));
-  const float PART1 = (4.f * mp2 * (GE * GE) + Q2 * (GM * GM)) / (4.f * mp2 + Q2);
-  const float DELTA = pt2 / (pt2 + xi2 * mp2);
+  const float PART1 = fmaf(4.f * mp2, GE * GE, Q2 * (GM * GM)) / (4.f * mp2 + Q2);
+  const float DELTA = pt2 / fmaf(xi2, mp2, pt2);
   const float f = (float)(0.0072973525693 / GRA_PI * 16.0 * GRA_PI * GRA_PI) *
-                  ((1.f - xi) * (DELTA * DELTA) * PART1 + (xi2 / 4.f) * DELTA * (GM * GM));
+                  fmaf((xi2 / 4.f) * DELTA, GM * GM, (1.f - xi) * (DELTA * DELTA) * PART1);
   return f / (xi * pt2);
 }
 __device__ __forceinline__ cxf photo_prop32(const RunParams& P, float s, float t, float B0) {

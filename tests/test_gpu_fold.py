@@ -107,3 +107,28 @@ def test_folded_nodes(name):
     sys.stdout.flush()
     assert np.array_equal(fg, fo) and np.all(Wg[~ok] == 0)
     assert ok.any() and rel.max() <= RTOL
+
+
+@pytest.mark.parametrize("name", sorted(RES_CASES))
+def test_folded_nodes_fp32_amplitude(name):
+    """The FP32-amplitude resonance nodes on folded kinematics, against the FP64 oracle.
+    Bound: an FP32 rounding is 6e-8, a node runs some tens of them on its largest terms,
+    and the screened amplitude can be 1/10 of its parts, squared: 6e-8 x 50 x 20 = 6e-5,
+    on the weights that FP32 resolves (above 1e-8 of the largest)."""
+    over, change = RES_CASES[name]
+    cfg = small_tables(abi.cfg_default(7), 500)
+    for key, value in over.items():
+        setattr(cfg, key, value)
+    if change:
+        change(cfg)
+    ref = abi.GraCfg.from_buffer_copy(cfg)
+    cfg.amp_precision, ref.amp_precision = abi.GRA_AMP_FP32, abi.GRA_AMP_FP64
+    print(f"case: {name}, FP32 amplitude, 65 points", flush=True)
+    u = np.random.default_rng(72).random((65, cfg.dim))
+    with MContinuum(cfg) as P:
+        Wg, _, fg = P.eval(u)
+    Wo, _, fo = ol.OracleRun(ref).eval(u)
+    big = Wo > 1e-8 * Wo.max()
+    rel = np.abs(Wg[big] - Wo[big]) / Wo[big]
+    print(f"{big.sum()} weights, max rel {rel.max():.2e}", flush=True)
+    assert np.array_equal(fg, fo) and rel.max() <= 6e-5
