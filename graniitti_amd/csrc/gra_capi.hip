@@ -14,6 +14,7 @@
 
 #include "gra_internal.h"
 #include "gra_kernels.h"
+#include "gra_round15.h"
 
 namespace gra_hip {
 
@@ -128,13 +129,6 @@ hcx interp_rows(const std::vector<double>& T, int N, double MIN, double STEP, do
   const double dx = x1 - x0;
   const hcx q = {(y1.re - y0.re) / dx, (y1.im - y0.im) / dx};
   return {y0.re + q.re * (a - x0), y0.im + q.im * (a - x0)};
-}
-
-// IArray1D::WriteArray / ReadArray round trip (std::setprecision(15), std::stod)
-double round15(double v) {
-  char buf[64];
-  snprintf(buf, sizeof(buf), "%.15g", v);
-  return std::strtod(buf, nullptr);
 }
 
 double gev2barn() {
