@@ -481,19 +481,14 @@ void fold_res_table(const gra_cfg& c, const std::vector<ResDev>& tab, FoldResTab
 // (beams below about 1.5 TeV, pairs at very large rapidity) keep the reference-order
 // nodes.
 bool fold_process(const gra_cfg& c, const RunParams& P) {
-  if (!c.screening || P.asym) return false;
+  if (!c.screening || P.asym || P.regge_k < 0) return false;
+  // the FP32 continuum has a node of its own
+  if (c.process == GRA_PROC_REGGE_CON && c.amp_precision != GRA_AMP_FP64) return false;
   // the component form's rounding differs from node to node and averages over a loop:
   // with a few nodes it stays at 3e-10 of the weight, and there is little to gain
   if (P.n_fold < 64) return false;
-  if (c.process == GRA_PROC_TENSOR_CON) {
-    // the FP32 node of the vector-meson pair
-    if (P.tp_mode != kTp2xV || c.amp_precision != GRA_AMP_FP32) return false;
-  } else {
-    if (P.regge_k < 0 || c.w_central > 0.0 || c.offshellFF != 2) return false;
-    // the FP32 continuum has a node of its own
-    if (c.process == GRA_PROC_REGGE_CON && c.amp_precision != GRA_AMP_FP64) return false;
-  }
-  if (c.process == GRA_PROC_RES_CON || c.process == GRA_PROC_RES) {
+  if (c.process == GRA_PROC_TENSOR_CON || c.w_central > 0.0 || c.offshellFF != 2) return false;
+  if (c.process != GRA_PROC_REGGE_CON) {
     // resonances: the Gottfried-Jackson axis moves with the node, the photon terms take
     // trajectory 0, and the traces are those of diagonal densities
     if (c.spin_frame == GRA_FRAME_GJ) return false;
@@ -507,8 +502,7 @@ bool fold_process(const gra_cfg& c, const RunParams& P) {
     E5 = std::hypot(P.f_Mmax, 2.0 * pT) * std::cosh(y);
   } else {
     const double kt = std::max(std::fabs(c.kt_min), std::fabs(c.kt_max));
-    const double m = c.m_central + c.offshell * c.w_central;  // GetOffShellMass's window
-    E5 = 2.0 * std::hypot(m, 0.5 * kt + pT) * std::cosh(y);
+    E5 = 2.0 * std::hypot(c.m_central, 0.5 * kt + pT) * std::cosh(y);
   }
   if (!(E5 < 0.2 * P.sqrt_s)) return false;
   const double b = 1.1 * c.m_beam * c.m_beam + (pT + km) * (pT + km);
