@@ -11,27 +11,86 @@ using gra_hip::kIterScalars;
 // Deterministic accumulation of one iteration. Each block owns a contiguous
 // range of points and has kAccWaves waves that walk the same points; wave w
 // owns the dimensions w, w + kAccWaves, ... and keeps their histograms of f and
-// f^2 in its own LDS slice. For each batch of 64 points and each owned
-// dimension the wave sorts the keys (bin, lane) with a bitonic network, sums f
-// and f^2 over each run of equal bins with a segmented scan, and the last lane
-// of each run adds the run's sums to its bin. Keys are unique, so the order of
-// every addition is fixed and the histograms are the same on every run, without
+// f^2 in its own LDS slice. For each batch of 64 points and each owned dimension
+// seven ballots, one a bit of the bin, give every lane the mask of the lanes that
+// share its bin; f and f^2 are summed over these by doubling the distance to the lane
+// before, and the last of them adds the sums to its bin. The order of every addition
+// is fixed by the points, so the histograms are the same on every run, without
 // atomics. Wave 0 also sums the scalars.
+// Bins are uniform on the VEGAS map, so 64 points put at most about four in one of 128
+// bins and two doublings do, at most six. Bound by instruction issue: about 300 a batch
+// for two dimensions, with the next batch's loads in flight; three waits in a row for W,
+// flags and bins made 2^20 points in 8 dimensions 43 us, now 36. Sorting (bin, lane) keys
+// with a bitonic network and scanning runs of equal bins took 97: 54 lane exchanges a
+// batch and dimension for 12 here. 80 registers; a bound of 64 for full occupancy spills
+// the time back (65 us).
 constexpr int kAccWave = 64;
 constexpr int kAccWaves = 4;
 
-// Ascending bitonic sort of one int key per lane across the wave
-__device__ __forceinline__ int wave_sort(int key, int lane) {
-#pragma unroll
-  for (int k = 2; k <= kAccWave; k <<= 1) {
-#pragma unroll
-    for (int j = k >> 1; j > 0; j >>= 1) {
-      const int other = __shfl_xor(key, j);
-      const bool up = (lane & k) == 0, lower = (lane & j) == 0;
-      key = (lower == up) ? min(key, other) : max(key, other);
+// The scalars of one iteration: sums with their compensations (value fs - fc), maxima, counts
+struct IterScal {
+  double fs = 0, fc = 0, f2s = 0, f2c = 0, mW = 0, mf = 0;
+  uint64_t kin = 0, fid = 0, val = 0, nan = 0, inf = 0;
+  // (s, c) += (os, oc): two-sum of the sums, carrying the compensations
+  static __device__ __forceinline__ void merge(double& s, double& c, double os, double oc) {
+    const double t = s + os, bp = t - s, e = (s - (t - bp)) + (os - bp);
+    s = t;
+    c = c + oc - e;
+  }
+  __device__ __forceinline__ void add(const double* p) {
+    merge(fs, fc, p[0], p[1]);
+    merge(f2s, f2c, p[2], p[3]);
+    mW = p[4] > mW ? p[4] : mW;
+    mf = p[5] > mf ? p[5] : mf;
+    kin += (uint64_t)p[6];
+    fid += (uint64_t)p[7];
+    val += (uint64_t)p[8];
+    nan += (uint64_t)p[9];
+    inf += (uint64_t)p[10];
+  }
+  // Over the wave in a fixed lane order, into lane 0
+  __device__ __forceinline__ void reduce() {
+    for (int off = kAccWave / 2; off > 0; off >>= 1) {
+      const double ofs = __shfl_down(fs, off), ofc = __shfl_down(fc, off);
+      const double of2s = __shfl_down(f2s, off), of2c = __shfl_down(f2c, off);
+      merge(fs, fc, ofs, ofc);
+      merge(f2s, f2c, of2s, of2c);
+      const double omW = __shfl_down(mW, off), omf = __shfl_down(mf, off);
+      mW = omW > mW ? omW : mW;
+      mf = omf > mf ? omf : mf;
+      kin += __shfl_down(kin, off);
+      fid += __shfl_down(fid, off);
+      val += __shfl_down(val, off);
+      nan += __shfl_down(nan, off);
+      inf += __shfl_down(inf, off);
     }
   }
-  return key;
+  __device__ __forceinline__ void store(double* o) const {
+    o[0] = fs;
+    o[1] = fc;
+    o[2] = f2s;
+    o[3] = f2c;
+    o[4] = mW;
+    o[5] = mf;
+    o[6] = (double)kin;
+    o[7] = (double)fid;
+    o[8] = (double)val;
+    o[9] = (double)nan;
+    o[10] = (double)inf;
+  }
+};
+
+// The lanes of the mask act whose 7-bit bin is this lane's
+__device__ __forceinline__ uint64_t wave_match(int bin, uint64_t act) {
+  uint32_t lo = (uint32_t)act, hi = (uint32_t)(act >> 32);
+#pragma unroll
+  for (int k = 0; k < 7; ++k) {
+    const int sign = (bin << (31 - k)) >> 31;  // all ones where the bit is set
+    const uint64_t set = __ballot(sign < 0);
+    lo &= ~((uint32_t)set ^ (uint32_t)sign);
+    hi &= ~((uint32_t)(set >> 32) ^ (uint32_t)sign);
+  }
+  return (uint64_t)hi << 32 | lo;
 }
 
 template <int DT>
@@ -41,78 +100,101 @@ __global__ __launch_bounds__(kAccWave* kAccWaves) void k_accumulate(
     double* __restrict__ part_hist, double* __restrict__ part_scal) {
   constexpr int DPW = (DT + kAccWaves - 1) / kAccWaves;  // dimensions per wave
   constexpr int NB = GRA_VEGAS_BINS;
-  __shared__ double hist[kAccWaves][DPW][2][NB];
+  static_assert(NB == 128, "wave_match compares seven bits");
+  __shared__ double2 hist[kAccWaves][DPW][NB];
   const int lane = threadIdx.x & (kAccWave - 1);
   const int wave = threadIdx.x / kAccWave;  // wave-uniform
-  double(*hw)[2][NB] = hist[wave];
+  double2(*hw)[NB] = hist[wave];
 #pragma unroll
   for (int q = 0; q < DPW; ++q)
-    for (int b = lane; b < NB; b += kAccWave) hw[q][0][b] = hw[q][1][b] = 0.0;
+    for (int b = lane; b < NB; b += kAccWave) hw[q][b] = make_double2(0.0, 0.0);
   const uint64_t p0 = (uint64_t)blockIdx.x * chunk;
   uint64_t p1 = p0 + chunk;
   if (p1 > n) p1 = n;
-  double fs = 0, fc = 0, f2s = 0, f2c = 0, mW = 0, mf = 0;
-  uint64_t c_kin = 0, c_fid = 0, c_val = 0, c_nan = 0, c_inf = 0;
+  IterScal scal;
+  struct Batch {
+    double W, vw;
+    uint8_t fl, bin[DPW];
+  };
+  // the lane's point of a batch; a lane past the last reads the last point again, a
+  // dimension past the last the last dimension
+  const auto load = [&](uint64_t base, Batch& v) {
+    const uint64_t i = min(base + lane, p1 - 1);
+    v.W = W[i];
+    v.vw = vw[i];
+    v.fl = flags[i];
+#pragma unroll
+    for (int q = 0; q < DPW; ++q) v.bin[q] = bins[i * D + min(wave + q * kAccWaves, D - 1)];
+  };
+  Batch next;
+  if (p0 < p1) load(p0, next);
   for (uint64_t base = p0; base < p1; base += kAccWave) {
-    const uint64_t i = base + lane;
-    double f = 0.0;
-    int bb[DPW];
-#pragma unroll
-    for (int q = 0; q < DPW; ++q) bb[q] = 0;
-    if (i < p1) {
-      const double Wi = W[i];
-      f = Wi * vw[i];
-      if (wave == 0) {
-        const double f2 = f * f;
-        double y = f - fc, t = fs + y;
-        fc = (t - fs) - y;
-        fs = t;
-        y = f2 - f2c;
-        t = f2s + y;
-        f2c = (t - f2s) - y;
-        f2s = t;
-        mW = Wi > mW ? Wi : mW;
-        mf = f > mf ? f : mf;
-        const uint8_t fl = flags[i];
-        c_kin += (fl & GRA_FLAG_KIN_OK) ? 1 : 0;
-        c_fid += (fl & GRA_FLAG_FID_OK) ? 1 : 0;
-        c_val += ((fl & GRA_FLAG_KIN_OK) && (fl & GRA_FLAG_FID_OK) && (fl & GRA_FLAG_VETO_OK)) ? 1
-                                                                                           : 0;
-        const bool bad = !(fl & GRA_FLAG_AMP_OK);
-        c_nan += (bad && !(fl & GRA_FLAG_INF)) ? 1 : 0;
-        c_inf += (bad && (fl & GRA_FLAG_INF)) ? 1 : 0;
-      }
-#pragma unroll
-      for (int q = 0; q < DPW; ++q) {
-        const int j = wave + q * kAccWaves;
-        if (j < D) bb[q] = bins[i * D + j];
-      }
+    const Batch v = next;
+    if (base + kAccWave < p1) load(base + kAccWave, next);  // in flight while this one is summed
+    const bool in = base + lane < p1;
+    const double f = in ? v.W * v.vw : 0.0;
+    if (wave == 0 && in) {
+      const double f2 = f * f;
+      double y = f - scal.fc, t = scal.fs + y;
+      scal.fc = (t - scal.fs) - y;
+      scal.fs = t;
+      y = f2 - scal.f2c;
+      t = scal.f2s + y;
+      scal.f2c = (t - scal.f2s) - y;
+      scal.f2s = t;
+      scal.mW = v.W > scal.mW ? v.W : scal.mW;
+      scal.mf = f > scal.mf ? f : scal.mf;
+      const uint8_t fl = v.fl;
+      scal.kin += (fl & GRA_FLAG_KIN_OK) ? 1 : 0;
+      scal.fid += (fl & GRA_FLAG_FID_OK) ? 1 : 0;
+      scal.val += ((fl & GRA_FLAG_KIN_OK) && (fl & GRA_FLAG_FID_OK) && (fl & GRA_FLAG_VETO_OK)) ? 1
+                                                                                             : 0;
+      const bool bad = !(fl & GRA_FLAG_AMP_OK);
+      scal.nan += (bad && !(fl & GRA_FLAG_INF)) ? 1 : 0;
+      scal.inf += (bad && (fl & GRA_FLAG_INF)) ? 1 : 0;
     }
-    if (__ballot(f != 0.0) == 0) continue;  // wave-uniform
+    const uint64_t act = __ballot(f != 0.0);
+    if (act == 0) continue;  // wave-uniform
+    double s[DPW], s2[DPW];
+    int prev[DPW];  // the lane before in this lane's bin; its own where there is none
+    bool tail[DPW];
+    const uint64_t below = (1ull << lane) - 1;
+    bool more = false;
 #pragma unroll
     for (int q = 0; q < DPW; ++q) {
-      if (wave + q * kAccWaves >= D) break;  // wave-uniform
-      // zero contributions sort behind every bin (key >= 128 * 64) and are dropped
-      const int key = wave_sort(f != 0.0 ? (bb[q] << 6) | lane : (NB << 6) | lane, lane);
-      const int bin = key >> 6;
-      double s = __shfl(f, key & 63);
-      double s2 = s * s;
-      // segmented inclusive scan over runs of equal bins (sorted, so a run is contiguous)
+      s[q] = f;
+      s2[q] = f * f;
+      // zero contributions are dropped, and so are dimensions past the last
+      const bool on = f != 0.0 && wave + q * kAccWaves < D;
+      const uint64_t same = wave_match(v.bin[q], act);
+      tail[q] = on && (same >> lane) == 1;
+      prev[q] = on && (same & below) ? 63 - __clzll(same & below) : lane;
+      more |= prev[q] != lane;
+    }
+    while (__ballot(more) != 0) {  // six times at most
+      more = false;
 #pragma unroll
-      for (int d = 1; d < kAccWave; d <<= 1) {
-        const int ob = __shfl_up(bin, d);
-        const double os = __shfl_up(s, d), os2 = __shfl_up(s2, d);
-        if (lane >= d && ob == bin) {
-          s += os;
-          s2 += os2;
+      for (int q = 0; q < DPW; ++q) {
+        const double os = __shfl(s[q], prev[q]), os2 = __shfl(s2[q], prev[q]);
+        const int op = __shfl(prev[q], prev[q]);
+        if (prev[q] != lane) {
+          s[q] += os;
+          s2[q] += os2;
         }
-      }
-      const int nb = __shfl_down(bin, 1);
-      if (bin < NB && (lane == kAccWave - 1 || nb != bin)) {
-        hw[q][0][bin] += s;
-        hw[q][1][bin] += s2;
+        // past the first of the bin's lanes there is no lane to add
+        prev[q] = op != prev[q] ? op : lane;
+        more |= prev[q] != lane;
       }
     }
+#pragma unroll
+    for (int q = 0; q < DPW; ++q)
+      if (tail[q]) {
+        const double2 h = hw[q][v.bin[q]];
+        hw[q][v.bin[q]] = make_double2(h.x + s[q], h.y + s2[q]);
+      }
+    // the next batch's lanes read what this one's wrote
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
   }
   const uint64_t H = 2 * (uint64_t)D * NB;
   double* ph = part_hist + (uint64_t)blockIdx.x * H;
@@ -121,98 +203,68 @@ __global__ __launch_bounds__(kAccWave* kAccWaves) void k_accumulate(
     const int j = wave + q * kAccWaves;
     if (j < D)
       for (int b = lane; b < NB; b += kAccWave) {
-        ph[j * NB + b] = hw[q][0][b];
-        ph[(D + j) * NB + b] = hw[q][1][b];
+        ph[j * NB + b] = hw[q][b].x;
+        ph[(D + j) * NB + b] = hw[q][b].y;
       }
   }
   if (wave != 0) return;
-  // Wave reduction of the scalars in a fixed lane order
-  for (int off = 32; off > 0; off >>= 1) {
-    const double ofs = __shfl_down(fs, off), ofc = __shfl_down(fc, off);
-    const double of2s = __shfl_down(f2s, off), of2c = __shfl_down(f2c, off);
-    // two-sum of the partial sums, carrying the compensations
-    double s = fs + ofs, bp = s - fs, e = (fs - (s - bp)) + (ofs - bp);
-    fs = s;
-    fc = fc + ofc - e;
-    s = f2s + of2s;
-    bp = s - f2s;
-    e = (f2s - (s - bp)) + (of2s - bp);
-    f2s = s;
-    f2c = f2c + of2c - e;
-    const double omW = __shfl_down(mW, off), omf = __shfl_down(mf, off);
-    mW = omW > mW ? omW : mW;
-    mf = omf > mf ? omf : mf;
-    c_kin += __shfl_down(c_kin, off);
-    c_fid += __shfl_down(c_fid, off);
-    c_val += __shfl_down(c_val, off);
-    c_nan += __shfl_down(c_nan, off);
-    c_inf += __shfl_down(c_inf, off);
-  }
-  if (lane == 0) {
-    double* o = part_scal + (uint64_t)blockIdx.x * kIterScalars;
-    o[0] = fs;
-    o[1] = fc;
-    o[2] = f2s;
-    o[3] = f2c;
-    o[4] = mW;
-    o[5] = mf;
-    o[6] = (double)c_kin;
-    o[7] = (double)c_fid;
-    o[8] = (double)c_val;
-    o[9] = (double)c_nan;
-    o[10] = (double)c_inf;
-  }
+  scal.reduce();
+  if (lane == 0) scal.store(part_scal + (uint64_t)blockIdx.x * kIterScalars);
 }
 
-// Fixed-order two-level reduction of the block partials. Stage 1: group g sums
-// blocks [g nblk / G, (g + 1) nblk / G) in order; stage 2 sums the groups in
-// order into gra_iter_stats layout: out[0 .. kIterScalars - 1] scalars, then the
-// histograms [2][D][128].
+// Reduction of the nblk block partials in a fixed order into gra_iter_stats layout:
+// out[0 .. kIterScalars - 1] scalars, then the histograms [2][D][128]. A block takes
+// kRedCols columns (128 bytes of each row): group g of kRedGroups sums the partials
+// [g nblk / G, (g + 1) nblk / G) of a column in order, then the groups are summed in
+// order. The block past the last column reduces the scalars. Bound by reading the
+// partials once, 16 loads of a thread in flight: 9 us for 2^20 points (2048 partials,
+// 34 MB), where two launches with a load at a time took 29 + 7; 6 us, a chain of waits,
+// for small passes.
+constexpr int kRedCols = 16;
 constexpr int kRedGroups = 32;
 
-// Kahan-add of one block's (sum, compensation) pair and the other scalars
-__device__ __forceinline__ void scal_add(double* a, const double* p) {
-  double y = (p[0] - p[1]) - a[1], tt = a[0] + y;
-  a[1] = (tt - a[0]) - y;
-  a[0] = tt;
-  y = (p[2] - p[3]) - a[3];
-  tt = a[2] + y;
-  a[3] = (tt - a[2]) - y;
-  a[2] = tt;
-  a[4] = p[4] > a[4] ? p[4] : a[4];
-  a[5] = p[5] > a[5] ? p[5] : a[5];
-  for (int k = 6; k < kIterScalars; ++k) a[k] += p[k];
-}
-
-__global__ void k_reduce1(const double* __restrict__ part_hist, const double* __restrict__ part_scal,
-                          int nblk, int H, double* __restrict__ tmp, double* __restrict__ tmp_scal) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  const int g = blockIdx.y;
-  const int b0 = (int)((long long)nblk * g / kRedGroups);
-  const int b1 = (int)((long long)nblk * (g + 1) / kRedGroups);
-  if (t < H) {
+__global__ __launch_bounds__(kRedCols* kRedGroups) void k_reduce(
+    const double* __restrict__ part_hist, const double* __restrict__ part_scal, int nblk, int H,
+    double* __restrict__ out) {
+  __shared__ double sum[kRedGroups][kRedCols];
+  __shared__ double sums[kRedCols * kRedGroups / kAccWave][kIterScalars];
+  const int t = threadIdx.x;
+  if ((int)blockIdx.x * kRedCols < H) {  // block-uniform; H is a multiple of kRedCols
+    const int c = t % kRedCols, g = t / kRedCols;
+    const int b0 = (int)((long long)nblk * g / kRedGroups);
+    const int b1 = (int)((long long)nblk * (g + 1) / kRedGroups);
+    const double* p = part_hist + (uint64_t)blockIdx.x * kRedCols + c;
     double s = 0.0;
-    for (int b = b0; b < b1; ++b) s += part_hist[(uint64_t)b * H + t];
-    tmp[(uint64_t)g * H + t] = s;
-  } else if (t == H) {
-    double a[kIterScalars] = {};
-    for (int b = b0; b < b1; ++b) scal_add(a, part_scal + (uint64_t)b * kIterScalars);
-    for (int k = 0; k < kIterScalars; ++k) tmp_scal[g * kIterScalars + k] = a[k];
+    int b = b0;
+    for (; b + 16 <= b1; b += 16) {
+      double v[16];
+#pragma unroll
+      for (int k = 0; k < 16; ++k) v[k] = p[(uint64_t)(b + k) * H];
+#pragma unroll
+      for (int k = 0; k < 16; ++k) s += v[k];
+    }
+    for (; b < b1; ++b) s += p[(uint64_t)b * H];
+    sum[g][c] = s;
+    __syncthreads();
+    if (g != 0) return;
+    s = 0.0;
+#pragma unroll
+    for (int k = 0; k < kRedGroups; ++k) s += sum[k][c];
+    out[kIterScalars + blockIdx.x * kRedCols + c] = s;
+    return;
   }
-}
-
-__global__ void k_reduce2(const double* __restrict__ tmp, const double* __restrict__ tmp_scal, int H,
-                          double* __restrict__ out) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < H) {
-    double s = 0.0;
-    for (int g = 0; g < kRedGroups; ++g) s += tmp[(uint64_t)g * H + t];
-    out[kIterScalars + t] = s;
-  } else if (t == H) {
-    double a[kIterScalars] = {};
-    for (int g = 0; g < kRedGroups; ++g) scal_add(a, tmp_scal + g * kIterScalars);
-    for (int k = 0; k < kIterScalars; ++k) out[k] = a[k];
-  }
+  const int lane = t & (kAccWave - 1), wave = t / kAccWave;
+  IterScal a;
+  for (int b = t; b < nblk; b += kRedCols * kRedGroups)
+    a.add(part_scal + (uint64_t)b * kIterScalars);
+  a.reduce();
+  if (lane == 0) a.store(sums[wave]);
+  __syncthreads();
+  if (wave != 0) return;
+  IterScal w;
+  if (lane < kRedCols * kRedGroups / kAccWave) w.add(sums[lane]);
+  w.reduce();
+  if (lane == 0) w.store(out);
 }
 
 // Map only (tests of the VEGAS map)
@@ -485,12 +537,8 @@ hipError_t launch_accumulate(const double* W, const double* vw, const uint8_t* b
     hipLaunchKernelGGL(k_accumulate<16>, dim3(nblk), dim3(kAccWave * kAccWaves), 0, st, W, vw,
                        bins, flags, n, chunk, D, part_hist, part_scal);
   const int H = 2 * D * GRA_VEGAS_BINS;
-  // stage-1 partial sums use the tail of part_hist's allocation: [G][H] then [G][kIterScalars]
-  double* tmp = part_hist + (uint64_t)nblk * H;
-  double* tmp_scal = tmp + (uint64_t)kRedGroups * H;
-  hipLaunchKernelGGL(k_reduce1, dim3((H + 1 + 255) / 256, kRedGroups), dim3(256), 0, st,
-                     part_hist, part_scal, nblk, H, tmp, tmp_scal);
-  hipLaunchKernelGGL(k_reduce2, dim3((H + 1 + 255) / 256), dim3(256), 0, st, tmp, tmp_scal, H, out);
+  hipLaunchKernelGGL(k_reduce, dim3(H / kRedCols + 1), dim3(kRedCols * kRedGroups), 0, st, part_hist,
+                     part_scal, nblk, H, out);
   return hipGetLastError();
 }
 
