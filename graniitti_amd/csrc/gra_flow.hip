@@ -29,6 +29,8 @@
 #include "gra_kernels.h"
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
 namespace {
@@ -1174,15 +1176,23 @@ __global__ void k_adam(float* __restrict__ th, const float* __restrict__ g, floa
   th[i] -= lr * (mi * c1) / (sqrtf(vi * c2) + eps);
 }
 
-// W[Kin x N] (row-major, fp32) -> Wt16[N x Kin] and W16[Kin x N] (bf16)
+// W[Kin x N] (row-major, fp32) -> Wt16[N x Kin], W16[Kin x N] and, in the order in which
+// the lanes of the fused layer's MFMAs hold it, Wf16 (bf16): 1 KB blocks of 16 columns by
+// 32 rows, in a block lane l's eight values, rows 8 (l / 16) .. of column l % 16. N and Kin
+// are multiples of 64. A block is one contiguous load of a wave; out of Wt16 it was 16
+// half cache lines, and a product's lines (49 KB for three tiles of eight waves) did not
+// stay in the 32 KB L1 until the next load took their other halves.
 __global__ void k_weights_bf16(const float* __restrict__ W, int Kin, int N, __bf16* __restrict__ Wt16,
-                               __bf16* __restrict__ W16, float* __restrict__ Wt32) {
+                               __bf16* __restrict__ W16, __bf16* __restrict__ Wf16,
+                               float* __restrict__ Wt32) {
   const int idx = blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= Kin * N) return;
   const int k = idx / N, c = idx % N;
   const float w = W[idx];
   Wt16[(size_t)c * Kin + k] = (__bf16)w;
   W16[idx] = (__bf16)w;
+  const int lane = 16 * (k % 32 / 8) + c % 16;
+  Wf16[((size_t)(c / 16) * (Kin / 32) + k / 32) * 512 + 8 * lane + k % 8] = (__bf16)w;
   Wt32[(size_t)c * Kin + k] = w;
 }
 
@@ -1306,7 +1316,7 @@ __host__ __device__ constexpr int fused_waves(int H) {
 struct FusedLayer {
   const float* W1;            // [dA x H]
   const float* b1;            // [H]
-  const __bf16* wt[4];        // transposed weights of products 1..depth: [N_i x H]
+  const __bf16* wt[4];        // weights of products 1..depth in fragment order (Wf16)
   const float* bias[4];       // biases of products 1..depth
   __bf16* act_out[4];         // optional stores of activations 0..depth-1 ([n x H])
   float* prm_out;             // optional store of the spline parameters ([n x ldp])
@@ -1325,23 +1335,40 @@ __device__ __forceinline__ void product_tiles(const __bf16* sA, int lda,
   constexpr int MT = R / 16;
   const int lane = threadIdx.x & 63;
   const int kq = 8 * (lane >> 4);
+  // k-steps whose weights are loaded together: the whole product up to H = 128 (a training
+  // step of 2^18 points 3.39 -> 3.32 ms); at H = 256 two waves a SIMD gain nothing from it
+  constexpr int KS = H / 32, PK = KS <= 4 ? KS : 1;
 #pragma unroll
-  for (int k0 = 0; k0 < H; k0 += 32) {
-    bf16x8 a[MT], b[TT];
+  for (int k1 = 0; k1 < KS; k1 += PK) {
+    bf16x8 b[PK][TT];
 #pragma unroll
-    for (int t = 0; t < TT; ++t)
-      b[t] = *(const bf16x8*)(wt + (size_t)((nt0 + NW * t) * 16 + (lane & 15)) * H + k0 + kq);
+    for (int k = 0; k < PK; ++k)
 #pragma unroll
-    for (int m = 0; m < MT; ++m)
-      a[m] = *(const bf16x8*)(sA + (size_t)(16 * m + (lane & 15)) * lda + k0 + kq);
+      for (int t = 0; t < TT; ++t)
+        b[k][t] = *(const bf16x8*)(wt + (size_t)((nt0 + NW * t) * KS + k1 + k) * 512 + 8 * lane);
 #pragma unroll
-    for (int t = 0; t < TT; ++t)
+    for (int k = 0; k < PK; ++k) {
+      bf16x8 a[MT];
 #pragma unroll
       for (int m = 0; m < MT; ++m)
-        acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m], b[t], acc[m][t], 0, 0, 0);
+        a[m] = *(const bf16x8*)(sA + (size_t)(16 * m + (lane & 15)) * lda + 32 * (k1 + k) + kq);
+#pragma unroll
+      for (int t = 0; t < TT; ++t)
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+          acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[k][t], a[m], acc[m][t], 0, 0, 0);
+    }
   }
 }
 
+// Four floats at any float's address
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
+
+// The weights are the first operand of the MFMA, so a lane holds four neighbouring
+// columns of one row: bias, ReLU and rounding go to LDS as one 8-byte (activations) or
+// 16-byte (parameters) write, and to memory the same way, where the other order had four
+// writes of 2 or 4 bytes in four rows.
 template <int H, int R, int NW>
 __device__ __forceinline__ void fused_product(const __bf16* sA, int lda, const __bf16* __restrict__ wt,
                                               const float* __restrict__ bias, int tb, int N,
@@ -1357,7 +1384,10 @@ __device__ __forceinline__ void fused_product(const __bf16* sA, int lda, const _
     // them exist (wave-uniform)
     constexpr int MT = R / 16;
     const int nv = min(4, (ntiles - nt0 + NW - 1) / NW);
-    f32x4 acc[MT][4];
+    f32x4 acc[MT][4], bs[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+      bs[t] = *(const f32x4u*)(bias + (tb + nt0 + NW * min(t, nv - 1)) * 16 + 4 * (lane >> 4));
 #pragma unroll
     for (int m = 0; m < MT; ++m)
 #pragma unroll
@@ -1373,107 +1403,131 @@ __device__ __forceinline__ void fused_product(const __bf16* sA, int lda, const _
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       if (t >= nv) break;
-      const int nt = nt0 + NW * t;
-      const int cl = nt * 16 + (lane & 15), col = tb * 16 + cl;
-      const float bv = bias[col];
+      const int cl = (nt0 + NW * t) * 16 + 4 * (lane >> 4), col = tb * 16 + cl;
+      const f32x4 bv = bs[t];
 #pragma unroll
-      for (int m = 0; m < MT; ++m)
+      for (int m = 0; m < MT; ++m) {
+        const int row = 16 * m + (lane & 15);
+        f32x4 v;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int row = 16 * m + 4 * (lane >> 4) + r;
-          float v = acc[m][t][r] + bv;
-          if (out_layer) {
-            if (col >= nvalid) v = 0.f;
-            sP[row * ldpp + cl] = v;
-            if (gprm && row0 + row < n) gprm[(size_t)(row0 + row) * ldp + col] = v;
-          } else {
-            v = fmaxf(v, 0.f);
-            const __bf16 hv = (__bf16)v;
-            sOut[row * ldo + cl] = hv;
-            if (gact && row0 + row < n) gact[(size_t)(row0 + row) * H + col] = hv;
-          }
+        for (int r = 0; r < 4; ++r) v[r] = acc[m][t][r] + bv[r];
+        if (out_layer) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (col + r >= nvalid) v[r] = 0.f;
+          *(f32x4*)(sP + row * ldpp + cl) = v;
+          if (gprm && row0 + row < n) *(f32x4u*)(gprm + (size_t)(row0 + row) * ldp + col) = v;
+        } else {
+          bf16x4 hv;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) hv[r] = (__bf16)fmaxf(v[r], 0.f);
+          *(bf16x4*)(sOut + row * ldo + cl) = hv;
+          if (gact && row0 + row < n) *(bf16x4*)(gact + (size_t)(row0 + row) * H + col) = hv;
         }
+      }
     }
   }
 }
 
 // Bin of the inverse spline (sampling direction) for one (point, dimension):
 // the softmax of the width and height logits p[0..K), p[K..2K), and the first
-// bin k whose cumulative height passes z (the last bin otherwise). KT > 0 is a
-// compile-time K: the logits are read once into registers and the loops are
-// unrolled; KT = 0 loops over a runtime K. Both orders of operations are the
-// same, so both give the same bin and values.
-template <int KT>
+// bin k whose cumulative height passes z (the last bin otherwise). inverse_bin loops
+// over a runtime K. inverse_bin2 has K at compile time and two lanes a spline, 2 i and
+// 2 i + 1: the even one takes the widths, the odd one the heights, each its K logits in
+// registers from 16-byte reads; the bin goes to the even lane, which sums the widths
+// below it. One lane a spline left half the threads idle and took twice the exponentials
+// of the widths; the orders of operations are the same, and so are bin and values.
 __device__ __forceinline__ void inverse_bin(const float* p, int K, float zv, Bin& e) {
   float X = 0.f, Y = 0.f, w = 0.f, h = 0.f;
   int k = 0;
-  if constexpr (KT > 0) {
-    // heights in registers: their softmax and the bin search; the widths are
-    // then walked from LDS (two exponentials each) to keep the registers low
-    float eh[KT];
-#pragma unroll
-    for (int m = 0; m < KT; ++m) eh[m] = p[KT + m];
-    float mw = p[0], mh = eh[0];
-#pragma unroll
-    for (int m = 1; m < KT; ++m) {
-      mw = fmaxf(mw, p[m]);
-      mh = fmaxf(mh, eh[m]);
-    }
-    float sw = 0.f, sh = 0.f;
-#pragma unroll
-    for (int m = 0; m < KT; ++m) {
-      sw += __expf(p[m] - mw);
-      eh[m] = __expf(eh[m] - mh);
-      sh += eh[m];
-    }
-    const float cw = 1.f - KT * kEpsW;
-    const float iw = cw / sw, ih = cw / sh;
-    float Ya = 0.f;
-    bool found = false;
-#pragma unroll
-    for (int m = 0; m < KT; ++m) {
-      const float hm = kEpsW + eh[m] * ih;
-      const bool hit = !found && (m == KT - 1 || Ya + hm > zv);
-      k = hit ? m : k;
-      Y = hit ? Ya : Y;
-      h = hit ? hm : h;
-      found = found || hit;
-      Ya += hm;
-    }
-#pragma unroll
-    for (int m = 0; m < KT; ++m) {
-      const float wm = kEpsW + __expf(p[m] - mw) * iw;
-      w = (m == k) ? wm : w;
-      X = (m < k) ? X + wm : X;
-    }
-  } else {
-    float mw = p[0], mh = p[K];
-    for (int m = 1; m < K; ++m) {
-      mw = fmaxf(mw, p[m]);
-      mh = fmaxf(mh, p[K + m]);
-    }
-    float sw = 0.f, sh = 0.f;
-    for (int m = 0; m < K; ++m) {
-      sw += __expf(p[m] - mw);
-      sh += __expf(p[K + m] - mh);
-    }
-    const float cw = 1.f - K * kEpsW;
-    const float iw = cw / sw, ih = cw / sh;
-    for (; k < K; ++k) {
-      w = kEpsW + __expf(p[k] - mw) * iw;
-      h = kEpsW + __expf(p[K + k] - mh) * ih;
-      if (k == K - 1 || Y + h > zv) break;
-      X += w;
-      Y += h;
-    }
+  float mw = p[0], mh = p[K];
+  for (int m = 1; m < K; ++m) {
+    mw = fmaxf(mw, p[m]);
+    mh = fmaxf(mh, p[K + m]);
+  }
+  float sw = 0.f, sh = 0.f;
+  for (int m = 0; m < K; ++m) {
+    sw += __expf(p[m] - mw);
+    sh += __expf(p[K + m] - mh);
+  }
+  const float cw = 1.f - K * kEpsW;
+  const float iw = cw / sw, ih = cw / sh;
+  for (; k < K; ++k) {
+    w = kEpsW + __expf(p[k] - mw) * iw;
+    h = kEpsW + __expf(p[K + k] - mh) * ih;
+    if (k == K - 1 || Y + h > zv) break;
+    X += w;
+    Y += h;
   }
   e.k = k;
   e.X = X;
   e.w = w;
   e.Y = Y;
   e.h = h;
+  e.dk = (k == 0) ? 1.f : kEpsD + softplusf(p[2 * K + k - 1]);
+  e.dk1 = (k == K - 1) ? 1.f : kEpsD + softplusf(p[2 * K + k]);
 }
 
+template <int KT>
+__device__ __forceinline__ void inverse_bin2(const float* p, int odd, float zv, Bin& e) {
+  float v[KT];
+#pragma unroll
+  for (int m = 0; m < KT; m += 4) {
+    const f32x4 q = *(const f32x4*)(p + odd * KT + m);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[m + r] = q[r];
+  }
+  float mx = v[0];
+#pragma unroll
+  for (int m = 1; m < KT; ++m) mx = fmaxf(mx, v[m]);
+  float sum = 0.f;
+#pragma unroll
+  for (int m = 0; m < KT; ++m) {
+    v[m] = __expf(v[m] - mx);
+    sum += v[m];
+  }
+  const float cw = 1.f - KT * kEpsW;
+  const float inv = cw / sum;
+  // every term is at least kEpsW, so the sums grow and the bins below z come first
+  int k = 0;
+  float acc = 0.f;
+#pragma unroll
+  for (int m = 0; m < KT; ++m) {
+    v[m] = kEpsW + v[m] * inv;
+    acc += v[m];
+    if (m < KT - 1) k += !(acc > zv);
+  }
+  const int lane = threadIdx.x & 63, ev = lane & ~1, od = lane | 1;
+  k = __shfl(k, od);
+  // the sum below bin k and the term at k: X, w in the even lane, Y, h in the odd one
+  float below = 0.f, at = v[0];
+  acc = 0.f;
+#pragma unroll
+  for (int m = 0; m < KT - 1; ++m) {
+    acc += v[m];
+    below = m < k ? acc : below;
+    at = m < k ? v[m + 1] : at;
+  }
+  // the derivatives at the bin's ends, one a lane; 1 at the ends of [0, 1]
+  const bool end = odd ? k == KT - 1 : k == 0;
+  const float d = end ? 1.f : kEpsD + softplusf(p[2 * KT + (end ? 0 : k - 1 + odd)]);
+  e.k = k;
+  e.X = __shfl(below, ev);
+  e.w = __shfl(at, ev);
+  e.Y = __shfl(below, od);
+  e.h = __shfl(at, od);
+  e.dk = __shfl(d, ev);
+  e.dk1 = __shfl(d, od);
+}
+
+// One coupling layer in the sampling direction, 64 points a block: input layer, hidden and
+// output products on MFMA, spline inverses, all out of LDS. Bound by the phases around the
+// products, which barriers keep apart: a block at 3 x 256, K = 32 took 88000 cycles, 9000 of
+// them MFMA. Weights came in half cache lines that overflowed the L1 (24000 cycles), the
+// products went to LDS in four short writes for one long, the inputs were read from LDS one
+// by one, and the splines left half the threads idle: without these 52000, and less with
+// the shorter bin search. Bits unchanged. 10^5 points at 3 x 256, K = 32: 285 -> 143 us a
+// layer; 2^18 points at 2 x 128, K = 16, with the stores for training: 153 -> 119 us.
 template <int H, int KT>
 __global__ __launch_bounds__(fused_threads(H), fused_waves(H)) void k_flow_layer_inverse(
     const float* __restrict__ u_in, float* __restrict__ u_out, float* __restrict__ ld, int n,
@@ -1489,7 +1543,7 @@ __global__ __launch_bounds__(fused_threads(H), fused_waves(H)) void k_flow_layer
   __bf16* sY = sX + R * lda;
   float* sP = (float*)sY;
   const int ybytes = max(R * lda * (int)sizeof(__bf16), R * ldpp * (int)sizeof(float));
-  float* sLj = (float*)((unsigned char*)sY + ybytes);
+  float* sLj = (float*)((unsigned char*)sY + ybytes);  // the input layer's inputs, then log J
   float* sU = sLj + R * 8;  // the block's input rows [R x D]
   const int row0 = blockIdx.x * R;
   for (int e = threadIdx.x; e < R * D; e += blockDim.x) {
@@ -1501,28 +1555,46 @@ __global__ __launch_bounds__(fused_threads(H), fused_waves(H)) void k_flow_layer
   // reads X and writes the parameter tile over Y
   __bf16* cur = (depth & 1) ? sX : sY;
   __bf16* nxt = (depth & 1) ? sY : sX;
-  // input layer (FP32 VALU): act0 = relu(u[A] W1 + b1); each thread owns one
-  // column, with its weights in registers, for R / (NT / H) rows
+  // input layer (FP32 VALU): act0 = relu(u[A] W1 + b1); the rows' inputs gathered into
+  // eights, so a row is two 16-byte reads; each thread owns two neighbouring columns, with
+  // their weights in registers, for R / (2 NT / H) rows. Inputs past dA are column 0 with
+  // weight 0, so no load is conditional.
+  for (int i = threadIdx.x >> 6; i < kMaxDB; i += NT / 64) {
+    const int a = i < L.dA ? L.A[i] : 0;
+    for (int r = threadIdx.x & 63; r < R; r += 64) {
+      const float u = sU[r * D + a];
+      sLj[r * kMaxDB + i] = u;
+      if (i < L.dA && row0 + r < n) u_out[(size_t)(row0 + r) * D + a] = u;  // passed through
+    }
+  }
+  __syncthreads();
   {
-    constexpr int nrg = NT / H;
-    const int j = threadIdx.x % H, rg = threadIdx.x / H;
-    // indices past dA read column 0 with weight 0, so no load is conditional
-    float w[kMaxDB];
-    int ai[kMaxDB];
+    constexpr int nrg = 2 * NT / H;
+    const int j = 2 * (threadIdx.x % (H / 2)), rg = threadIdx.x / (H / 2);
+    float w0[kMaxDB], w1[kMaxDB];
 #pragma unroll
     for (int i = 0; i < kMaxDB; ++i) {
       const bool on = i < L.dA;
-      w[i] = on ? W.W1[(on ? i : 0) * H + j] : 0.f;
-      ai[i] = on ? L.A[i] : 0;
+      const f32x2u w = *(const f32x2u*)(W.W1 + (on ? i : 0) * H + j);
+      w0[i] = on ? w[0] : 0.f;
+      w1[i] = on ? w[1] : 0.f;
     }
-    const float bj = W.b1[j];
+    const float b0 = W.b1[j], b1 = W.b1[j + 1];
+#pragma unroll 4
     for (int r = rg; r < R; r += nrg) {
-      float acc = bj;
+      const f32x4 ua = *(const f32x4*)(sLj + r * kMaxDB), ub = *(const f32x4*)(sLj + r * kMaxDB + 4);
+      float x0 = b0, x1 = b1;
 #pragma unroll
-      for (int i = 0; i < kMaxDB; ++i) acc += sU[r * D + ai[i]] * w[i];
-      const __bf16 hv = (__bf16)fmaxf(acc, 0.f);
-      cur[r * lda + j] = hv;
-      if (W.act_out[0] && row0 + r < n) W.act_out[0][(size_t)(row0 + r) * H + j] = hv;
+      for (int i = 0; i < kMaxDB; ++i) {
+        const float u = i < 4 ? ua[i & 3] : ub[i & 3];
+        x0 += u * w0[i];
+        x1 += u * w1[i];
+      }
+      bf16x2 hv;
+      hv[0] = (__bf16)fmaxf(x0, 0.f);
+      hv[1] = (__bf16)fmaxf(x1, 0.f);
+      *(bf16x2*)(cur + r * lda + j) = hv;
+      if (W.act_out[0] && row0 + r < n) *(bf16x2*)(W.act_out[0] + (size_t)(row0 + r) * H + j) = hv;
     }
   }
   __syncthreads();
@@ -1546,20 +1618,23 @@ __global__ __launch_bounds__(fused_threads(H), fused_waves(H)) void k_flow_layer
                                  L.dB * nps, true, nxt, lda, sP, ldpp, nullptr, W.prm_out, row0, n,
                                  ldp);
     __syncthreads();
-    // (row, dimension) pairs of the group; R g may exceed the block's threads
-    for (int q = t; q < R * g; q += NT) {
-      const int r = q / g, j = j0 + q % g;
+    // (row, dimension) pairs of the group, rows fastest so that the lanes' parameters lie
+    // in different banks; two lanes a pair where K is known, the even one writes the point
+    constexpr int LP = KT > 0 ? 2 : 1;
+    const int odd = t % LP;
+    for (int q = t / LP; q < R * g; q += NT / LP) {
+      // a wave's pairs lie in one dimension
+      static_assert(R % (64 / LP) == 0, "q / R is uniform over the wave");
+      const int r = q % R, j = j0 + __builtin_amdgcn_readfirstlane(q / R);
       const int row = row0 + r;
       if (row >= n) continue;
-      if (j == 0)
-        for (int i = 0; i < L.dA; ++i) u_out[(size_t)row * D + L.A[i]] = sU[r * D + L.A[i]];
       const float* p = sP + r * ldpp + j * nps - 16 * tb;
       const float zv = fminf(fmaxf(sU[r * D + L.B[j]], 0.f), 1.f);
       Bin e;
-      inverse_bin<KT>(p, K, zv, e);
-      const int k = e.k;
-      e.dk = (k == 0) ? 1.f : kEpsD + softplusf(p[2 * K + k - 1]);
-      e.dk1 = (k == K - 1) ? 1.f : kEpsD + softplusf(p[2 * K + k]);
+      if constexpr (KT > 0)
+        inverse_bin2<KT>(p, odd, zv, e);
+      else
+        inverse_bin(p, K, zv, e);
       e.s = e.h / e.w;
       const float zeta = zv - e.Y;
       const float Dl = e.dk1 + e.dk - 2.f * e.s;
@@ -1571,15 +1646,16 @@ __global__ __launch_bounds__(fused_threads(H), fused_waves(H)) void k_flow_layer
       xi = fminf(fmaxf(xi, 0.f), 1.f);
       float zz, lj;
       rqs_value(e, xi, zz, lj);
-      u_out[(size_t)row * D + L.B[j]] = fminf(fmaxf(e.X + xi * e.w, 0.f), 0.99999994f);
-      sLj[r * 8 + j] = lj;
+      if (odd == 0)
+        u_out[(size_t)row * D + L.B[j]] = fminf(fmaxf(e.X + xi * e.w, 0.f), 0.99999994f);
+      if (odd == LP - 1) sLj[r * kMaxDB + j] = lj;
     }
     __syncthreads();
   }
   for (int r = t; r < R; r += NT) {
     if (row0 + r >= n) break;
     float acc = 0.f;
-    for (int jj = 0; jj < L.dB; ++jj) acc += sLj[r * 8 + jj];
+    for (int jj = 0; jj < L.dB; ++jj) acc += sLj[r * kMaxDB + jj];
     ld[row0 + r] += acc;
   }
 }
@@ -1618,7 +1694,7 @@ struct FlowState {
   std::vector<FlowLayerHost> layers;
   size_t nparam = 0;
   DevBuf theta, grad, adam_m, adam_v, frozen;
-  DevBuf wt16, w16, wt32;  // per layer, per GEMM weight (hidden and output)
+  DevBuf wt16, w16, wf16, wt32;  // per layer, per GEMM weight (hidden and output)
   std::vector<size_t> wofs;  // element offsets of each GEMM weight copy
   // batch buffers
   int cap = 0;
@@ -1630,7 +1706,7 @@ struct FlowState {
 
 void flow_release(FlowState* f) {
   if (!f) return;
-  DevBuf* b[] = {&f->theta, &f->grad,   &f->adam_m, &f->adam_v, &f->frozen, &f->wt16, &f->w16,
+  DevBuf* b[] = {&f->theta, &f->grad,   &f->adam_m, &f->adam_v, &f->frozen, &f->wt16, &f->w16, &f->wf16,
                  &f->wt32,  &f->z,      &f->us,     &f->ld,     &f->acts16, &f->acts32, &f->prm,
                  &f->gprm,  &f->gprm16, &f->dact16, &f->dact32, &f->gu0,    &f->gu1,   &f->coef,
                  &f->xx,    &f->vw,     &f->W,      &f->wts,    &f->part,   &f->tmp,   &f->dh32,
@@ -1752,7 +1828,8 @@ static int refresh_weights(gra_handle* h, FlowState* F) {
       const int n = F->H * N;
       hipLaunchKernelGGL(k_weights_bf16, dim3((n + 255) / 256), dim3(256), 0, h->stream,
                          F->theta.as<float>() + off, F->H, N, F->wt16.as<__bf16>() + F->wofs[slot],
-                         F->w16.as<__bf16>() + F->wofs[slot], F->wt32.as<float>() + F->wofs[slot]);
+                         F->w16.as<__bf16>() + F->wofs[slot], F->wf16.as<__bf16>() + F->wofs[slot],
+                         F->wt32.as<float>() + F->wofs[slot]);
       ++slot;
     }
   }
@@ -1979,7 +2056,7 @@ static void fused_groups(const FlowState* F, int dB, int want, int& gd, int& ldg
       const int j1 = std::min(dB, j0 + g);
       w = std::max(w, (j1 * nps + 15) / 16 - (j0 * nps) / 16);
     }
-    return 16 * w + 1;
+    return 16 * w + 4;  // rows on 16 bytes, eight of them over all banks
   };
   gd = want > 0 ? std::min(want, dB) : dB;
   if (want <= 0)
@@ -2011,7 +2088,7 @@ static int flow_sample_pass(gra_handle* h, FlowState* F, int n, uint64_t seed, u
       W.W1 = th + Ly.oW1;
       W.b1 = th + Ly.ob1;
       for (int i = 1; i <= F->depth; ++i) {
-        W.wt[i - 1] = F->wt16.as<__bf16>() + F->wofs[l * F->depth + i - 1];
+        W.wt[i - 1] = F->wf16.as<__bf16>() + F->wofs[l * F->depth + i - 1];
         W.bias[i - 1] = th + (i == F->depth ? Ly.obo : Ly.obh[i]);
       }
       if (store) {
@@ -2282,7 +2359,7 @@ extern "C" int gra_hip_flow_init(gra_handle* h, const gra_flow_cfg* fc_in) {
       wo += (size_t)F->H * ((i == F->depth) ? F->ldp : F->H);
     }
   if (F->theta.ensure(4 * off) || F->grad.ensure(4 * off) || F->adam_m.ensure(4 * off) ||
-      F->adam_v.ensure(4 * off) || F->frozen.ensure(off) || F->wt16.ensure(2 * wo) ||
+      F->adam_v.ensure(4 * off) || F->frozen.ensure(off) || F->wt16.ensure(2 * wo) || F->wf16.ensure(2 * wo) ||
       F->w16.ensure(2 * wo) || F->wt32.ensure(4 * wo)) {
     flow_release(F);
     return fail(h, GRA_E_NOMEM, "flow parameters");
