@@ -78,7 +78,7 @@ struct gra_handle {
 
   // per-point buffers
   gra_hip::DevBuf d_x, d_W, d_amp2, d_flags, d_vw, d_bins, d_rec, d_ncand, d_grid;
-  gra_hip::DevBuf d_part_hist, d_part_scal, d_stats, d_aux;
+  gra_hip::DevBuf d_part_hist, d_part_scal, d_aux;
   // generation passes: accepted indices, hit masks, tile counts/offsets, event
   // records (grow-only), and the pass counters in pinned host memory
   gra_hip::DevBuf d_gen_idx, d_gen_mask, d_gen_tile, d_gen_cnt, d_gen_ev;
@@ -86,7 +86,9 @@ struct gra_handle {
   // pinned staging of event records bound for pageable caller memory (grow-only)
   void* h_ev_stage = nullptr;
   size_t h_ev_stage_bytes = 0;
-  std::vector<double> h_stats;
+  // pinned memory that kernels read and write in place of copies (grow-only, bounded)
+  void* h_pin = nullptr;
+  size_t h_pin_bytes = 0;
   // the grid edges last copied to d_grid: consecutive generation passes draw from
   // one grid, which is then not copied again
   std::vector<double> grid_host;
