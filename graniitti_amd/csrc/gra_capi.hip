@@ -996,7 +996,7 @@ static void time_collect(gra_handle* h, bool tree, bool screen, bool accum) {
 }
 
 // The integrand kernels on the handle's stream: the tree stage appends the
-// points that need screening to rec through the counter ncand (zero on entry),
+// points that need screening to rec through the two counters ncand (zero on entry),
 // the screening stage completes them. timed: record the kernel durations.
 static int launch_integrand(gra_handle* h, const double* d_grid, unsigned int bins, uint64_t seed,
                             uint32_t iter, uint64_t first, const double* d_x, uint64_t n,
@@ -1025,7 +1025,7 @@ int run_integrand(gra_handle* h, const double* d_grid, unsigned int bins, uint64
                   uint32_t iter, uint64_t first, const double* d_x, uint64_t n, double* d_W,
                   double* d_amp2, uint8_t* d_flags, double* d_vw, uint8_t* d_bins) {
   uint32_t* ncand = h->d_ncand.as<uint32_t>();
-  if (h->P.screening) GRA_HIP_CHECK(h, hipMemsetAsync(ncand, 0, sizeof(uint32_t), h->stream));
+  if (h->P.screening) GRA_HIP_CHECK(h, hipMemsetAsync(ncand, 0, 2 * sizeof(uint32_t), h->stream));
   return launch_integrand(h, d_grid, bins, seed, iter, first, d_x, n, d_W, d_amp2, d_flags, d_vw,
                           d_bins, h->d_rec.p, ncand, true);
 }
@@ -1235,8 +1235,8 @@ extern "C" int gra_hip_eval_points_noalloc(gra_handle* h, const double* d_u, siz
   double* vw = (double*)(base + off);
   off += align256(sizeof(double) * n);
   uint8_t* bins = base + off;
-  // the counter is cleared by a kernel (no memset node, so the call can be captured)
-  GRA_HIP_CHECK(h, launch_fill_u32(ncand, 0u, 1, h->stream));
+  // the counters are cleared by a kernel (no memset node, so the call can be captured)
+  GRA_HIP_CHECK(h, launch_fill_u32(ncand, 0u, 2, h->stream));
   const int r = launch_integrand(h, nullptr, 0, 0, 0, 0, d_u, n, d_W, d_amp2, d_flags, vw, bins,
                                  rec, ncand, false);
   if (r) return r;

@@ -189,9 +189,11 @@ __device__ __forceinline__ double solvepz_b(double m3, double m4, double pt3, do
           pz5 * (a3 * (1.0 / 2.0) - a4 * (1.0 / 2.0) + a5 * (1.0 / 2.0) - a6 * (1.0 / 2.0))) /
              (s + a2 - a7 - E5 * rs * 2.0);
 }
+// The masses for which SolvePz takes its equal-mass form
+__device__ __forceinline__ bool equal_masses(double m3, double m4) { return fabs(m3 - m4) < 1e-9; }
 __device__ __forceinline__ double solvepz(double m3, double m4, double pt3, double pt4, double pz5,
                                           double E5, const RunParams& P) {
-  if (fabs(m3 - m4) < 1e-9) return solvepz_a(m3, pt3, pt4, pz5, E5, P.s, P.rs, P.s32);
+  if (equal_masses(m3, m4)) return solvepz_a(m3, pt3, pt4, pz5, E5, P.s, P.rs, P.s32);
   return solvepz_b(m3, m4, pt3, pt4, pz5, E5, P.s, P.rs, P.s32);
 }
 
