@@ -88,36 +88,6 @@ hcx regge_eta(double alpha_t, double sigma) {
   return {-num.re / denom, -num.im / denom};
 }
 
-double s3f(const gra_cfg& c, double t) { return (1.0 / (1 - t / c.fc1)) * (1.0 / (1 - t / c.fc2)); }
-
-// form::S3HPL and form::S3PomAlpha, src/MForm.cc:402-426
-double s3hpl(const gra_cfg& c, double tau, double t) {
-  const double m = 1.0;
-  const double sqrtau = msqrt(1 + tau);
-  const double F_pi = 1.0 / (1.0 - t / c.fc3);
-  const double mpi = c.mpi_const;
-  return (4.0 / tau) * (F_pi * F_pi) *
-         (2.0 * tau - std::pow(1.0 + tau, 3.0 / 2.0) * std::log((sqrtau + 1.0) / (sqrtau - 1.0)) +
-          std::log((m * m) / (mpi * mpi)));
-}
-double pom_alpha(const gra_cfg& c, double t) {
-  const double mpi = c.mpi_const;
-  const double BETApi = (2.0 / 3.0) * c.gN_P;
-  const double PIC = ((BETApi * BETApi) * (mpi * mpi)) / (32.0 * (GRA_PI * (GRA_PI * GRA_PI)));
-  const double h = PIC * s3hpl(c, 4.0 * (mpi * mpi) / std::fabs(t), t);
-  return 1.0 + c.delta_P + c.alpha_P * t - h;
-}
-
-// MEikonal::SingleAmpElastic(s, t, +1), src/MEikonal.cc:139-154
-hcx single_amp_elastic(const gra_cfg& c, double s, double t) {
-  const double F = s3f(c, t);
-  const double aP = pom_alpha(c, t);
-  const hcx eta = regge_eta(aP, 1);
-  const double pre = ((c.gN_P * c.gN_P) * F) * F;
-  const double pw = std::pow(s / 1.0, aP);
-  return {(eta.re * pre) * pw, (eta.im * pre) * pw};
-}
-
 // IArray1D::Interpolate1D on rows (x, re, im), src/MEikonal.cc:489-512
 hcx interp_rows(const std::vector<double>& T, int N, double MIN, double STEP, double a) {
   if (a < MIN) a = MIN;
@@ -712,24 +682,18 @@ int build_eikonal(gra_handle* h, const char* cache_dir) {
   const gra_cfg& c = h->cfg;
   const RunParams& P = h->P;
   const int NF = c.n_fb;
-  std::vector<double> pre(2 * (size_t)(NF + 1));
-  DevBuf d_pre, d_out;
+  DevBuf d_pre, d_out, d_mbt;
   const int nrow_max = std::max(std::max(c.n_bt, c.n_kt2) + 1, c.eik_log_nodes);
-  if (d_pre.ensure(sizeof(double) * pre.size()) || d_out.ensure(sizeof(double) * 2 * nrow_max))
+  if (d_pre.ensure(sizeof(double) * 2 * (NF + 1)) || d_out.ensure(sizeof(double) * 2 * nrow_max))
     return fail(h, GRA_E_NOMEM, "eikonal table buffers");
   std::vector<double> out(2 * (size_t)nrow_max);
   // Density Omega(bt): pre_q = SingleAmpElastic(s, -kt_q^2)
   const double kmin = 1E-9, kmax = 30.0, kstep = (kmax - kmin) / NF;
-  for (int q = 0; q <= NF; ++q) {
-    const double kt = kmin + q * kstep;
-    const hcx a = single_amp_elastic(c, P.s, -(kt * kt));
-    pre[2 * q] = a.re;
-    pre[2 * q + 1] = a.im;
-  }
   const double bmin = 1E-6, bmax = 10.0 / gev2fm(), bstep = (bmax - bmin) / c.n_bt;
   int r = cached_table(h, cache_dir, 0, c.n_bt + 1, h->mbt, [&]() -> int {
-    GRA_HIP_CHECK(h, hipMemcpyAsync(d_pre.p, pre.data(), sizeof(double) * pre.size(),
-                                    hipMemcpyHostToDevice, h->stream));
+    const ElasticAmp A = {P.s,   c.gN_P,      c.fc1,     c.fc2,
+                          c.fc3, c.mpi_const, c.delta_P, c.alpha_P};
+    GRA_HIP_CHECK(h, launch_density_pre(A, NF, kmin, kstep, d_pre.as<double>(), h->stream));
     GRA_HIP_CHECK(h, launch_fb_table(0, d_pre.as<double>(), NF, kmin, kstep, bmin, bstep,
                                      c.n_bt + 1, 1 / (2.0 * GRA_PI * P.s), d_out.as<double>(),
                                      h->stream, nullptr));
@@ -747,19 +711,18 @@ int build_eikonal(gra_handle* h, const char* cache_dir) {
   if (r != GRA_OK) return r;
   // Screening amplitude A_eik(kt^2): pre_q = i (1 - exp(i Omega(bt_q) / 2))
   const double STEP = (bmax - bmin) / NF;
-  for (int q = 0; q <= NF; ++q) {
-    const double bt = bmin + q * STEP;
-    const hcx Om = interp_rows(h->mbt, c.n_bt, bmin, bstep, bt);
-    const hcx z = {(0.0 * Om.re - 1.0 * Om.im) / 2.0, (0.0 * Om.im + 1.0 * Om.re) / 2.0};
-    const hcx e = hexp(z);
-    const hcx om = {1.0 - e.re, -e.im};
-    pre[2 * q] = 0.0 * om.re - 1.0 * om.im;
-    pre[2 * q + 1] = 0.0 * om.im + 1.0 * om.re;
-  }
+  auto screening_pre = [&]() -> int {
+    const size_t bytes = sizeof(double) * h->mbt.size();
+    if (d_mbt.ensure(bytes)) return fail(h, GRA_E_NOMEM, "density table buffer");
+    GRA_HIP_CHECK(h, hipMemcpyAsync(d_mbt.p, h->mbt.data(), bytes, hipMemcpyHostToDevice, h->stream));
+    GRA_HIP_CHECK(h, launch_screening_pre(d_mbt.as<double>(), c.n_bt, bmin, bstep, NF, STEP,
+                                          d_pre.as<double>(), h->stream));
+    return GRA_OK;
+  };
   const double amin = 1E-6, amax = 25.0, astep = (amax - amin) / c.n_kt2;
   r = cached_table(h, cache_dir, 1, c.n_kt2 + 1, h->msa, [&]() -> int {
-    GRA_HIP_CHECK(h, hipMemcpyAsync(d_pre.p, pre.data(), sizeof(double) * pre.size(),
-                                    hipMemcpyHostToDevice, h->stream));
+    const int rp = screening_pre();
+    if (rp != GRA_OK) return rp;
     GRA_HIP_CHECK(h, launch_fb_table(1, d_pre.as<double>(), NF, bmin, STEP, amin, astep,
                                      c.n_kt2 + 1, (2.0 * P.s) * (2.0 * GRA_PI),
                                      d_out.as<double>(), h->stream, nullptr));
@@ -790,8 +753,8 @@ int build_eikonal(gra_handle* h, const char* cache_dir) {
     }
     DevBuf d_xs;
     if (d_xs.ensure(sizeof(double) * NL)) return fail(h, GRA_E_NOMEM, "log-node buffer");
-    GRA_HIP_CHECK(h, hipMemcpyAsync(d_pre.p, pre.data(), sizeof(double) * pre.size(),
-                                    hipMemcpyHostToDevice, h->stream));
+    r = screening_pre();
+    if (r != GRA_OK) return r;
     GRA_HIP_CHECK(h, hipMemcpyAsync(d_xs.p, xs.data(), sizeof(double) * NL, hipMemcpyHostToDevice,
                                     h->stream));
     GRA_HIP_CHECK(h, launch_fb_table(1, d_pre.as<double>(), NF, bmin, STEP, 0.0, 0.0, NL,
@@ -819,6 +782,7 @@ int build_eikonal(gra_handle* h, const char* cache_dir) {
   };
   d_pre.release();
   d_out.release();
+  d_mbt.release();
   // Loop nodes (phi_i, kt_j), i-major as the reference's (i, j) loops
   const int NP = c.n_loop_phi, NK = c.n_loop_kt;
   std::vector<double> gx, gw;

@@ -4,9 +4,12 @@
 #include <hip/hip_runtime.h>
 
 #include "gra_device.h"
+#include "gra_fold.h"
 #include "gra_kernels.h"
 
 namespace {
+
+using gra_hip::ElasticAmp;
 
 // J0 by the rational / asymptotic fits of Abramowitz-Stegun 9.4 as tabulated by
 // Clenshaw (NPL Math. Tables 5, 1962); the same approximation the reference
@@ -26,22 +29,76 @@ __device__ __forceinline__ double bessj0(double X) {
     const double FS = S1 + Y * (S2 + Y * (S3 + Y * (S4 + Y * (S5 + Y * S6))));
     return FR / FS;
   }
-  const double Z = 8.0 / AX;
+  // The fit's division, root and sincos as one reciprocal root and a reduction by
+  // quarter turns (exact in the first step: the difference is a multiple of 2^-52 below 1)
+  const double y = rsq64(AX);
+  const double Z = 8.0 * (y * y);
   const double Y = Z * Z;
   const double XX = AX - 0.785398164;
-  const double FP = P1 + Y * (P2 + Y * (P3 + Y * (P4 + Y * P5)));
-  const double FQ = Q1 + Y * (Q2 + Y * (Q3 + Y * (Q4 + Y * Q5)));
+  const double FP = __builtin_fma(Y, __builtin_fma(Y, __builtin_fma(Y, __builtin_fma(Y, P5, P4), P3), P2), P1);
+  const double FQ = __builtin_fma(Y, __builtin_fma(Y, __builtin_fma(Y, __builtin_fma(Y, Q5, Q4), Q3), Q2), Q1);
+  const double n = __builtin_rint(XX * 0.63661977236758138);
+  const double th = __builtin_fma(-n, 6.123233995736766e-17, __builtin_fma(-n, 1.5707963267948966, XX));
   double sn, cs;
-  sincos(XX, &sn, &cs);
-  return sqrt(0.636619772 / AX) * (FP * cs - Z * FQ * sn);
+  sincos_quarter64(n, th, sn, cs);
+  return 0.7978845605725179 * y * (FP * cs - Z * FQ * sn);  // sqrt(0.636619772 / AX) (..)
+}
+
+// The two integrands' factors at the quadrature nodes, a thread each; on the host these
+// loops (pow, log, exp and sincos at 10001 nodes each) took 0.7 of 3.4 ms of a set-up, here
+// 9 us.
+//
+// Density: pre_q = MEikonal::SingleAmpElastic(s, -kt_q^2), src/MEikonal.cc:139-154, with
+// form::S3HPL, S3PomAlpha and ReggeEta (src/MForm.cc:382-426)
+__global__ void k_density_pre(ElasticAmp A, int nf, double kmin, double kstep,
+                              double* __restrict__ pre) {
+  const int q = blockIdx.x * blockDim.x + threadIdx.x;
+  if (q > nf) return;
+  const double kt = kmin + q * kstep, t = -(kt * kt);
+  const double F = (1.0 / (1 - t / A.fc1)) * (1.0 / (1 - t / A.fc2));
+  const double mpi2 = A.mpi * A.mpi, beta = (2.0 / 3.0) * A.gN;
+  const double tau = 4.0 * mpi2 / fabs(t);
+  const double sqrtau = msq(1 + tau);
+  const double Fpi = 1.0 / (1.0 - t / A.fc3);
+  const double hpl = (4.0 / tau) * (Fpi * Fpi) *
+                     (2.0 * tau - pow(1.0 + tau, 1.5) * log((sqrtau + 1.0) / (sqrtau - 1.0)) +
+                      log(1.0 / mpi2));
+  const double pic = (beta * beta) * mpi2 / (32.0 * (GRA_PI * (GRA_PI * GRA_PI)));
+  const double alpha = 1.0 + A.delta + A.slope * t - pic * hpl;
+  double sn, cs;
+  sincos(GRA_PI * alpha, &sn, &cs);
+  const double a = ((A.gN * A.gN) * F) * F * pow(A.s, alpha);
+  pre[2 * q] = -((1.0 + cs) / sn) * a;  // eta = -(1 + exp(-i pi alpha)) / sin(pi alpha)
+  pre[2 * q + 1] = (sn / sn) * a;
+}
+// Screening: pre_q = i (1 - exp(i Omega(bt_q) / 2)), Omega between the density table's rows
+// (x, re, im) as IArray1D::Interpolate1D takes it (src/MEikonal.cc:489-512)
+__global__ void k_screening_pre(const double* __restrict__ T, int n_bt, double bmin, double bstep,
+                                int nf, double step, double* __restrict__ pre) {
+  const int q = blockIdx.x * blockDim.x + threadIdx.x;
+  if (q > nf) return;
+  double b = bmin + q * step;
+  if (b < bmin) b = bmin;
+  int i = (int)floor((b - bmin) / bstep);
+  i = min(max(i, 0), n_bt - 1);
+  const double* r = T + 3 * (size_t)i;
+  const double dx = r[3] - r[0], f = b - r[0];
+  const double re = r[1] + ((r[4] - r[1]) / dx) * f, im = r[2] + ((r[5] - r[2]) / dx) * f;
+  const double e = exp(-im / 2.0);
+  double sn, cs;
+  sincos(re / 2.0, &sn, &cs);
+  pre[2 * q] = e * sn;  // i (1 - e (cos + i sin))
+  pre[2 * q + 1] = 1.0 - e * cs;
 }
 
 // One wave per table row: lane l takes the quadrature nodes l, l + 64, ... (coalesced
 // loads, and the same Bessel branch across the wave but at one boundary), whose parity is
 // the lane's, and a butterfly adds the lanes' sums in a fixed order. With one thread per
 // row 10001 rows were 40 blocks, each a serial chain of 10001 terms: 6.0 ms a table at 16%
-// of the CUs. As waves they fill the chip, bound by the FP64 VALU (a division and a square
-// root or a sincos per term): 0.47 ms.
+// of the CUs. As waves they fill the chip, bound by the FP64 VALU: 0.52 ms with a division,
+// a library root and sincos a term (207 instructions), 0.33 with bessj0's (150). Against
+// 80-bit sums of the same fit the tables are off by 3e-15 of their largest value, as before
+// or less (screening 5.2e-15 and 2.9e-15 at 3.5 and 6.5 TeV beams, now 3.1e-15, 0.9e-15).
 constexpr int kFbWaves = 4;  // rows per block
 __global__ __launch_bounds__(64 * kFbWaves) void k_fb_table(int which, const double* __restrict__ pre, int nf,
                                                   double qmin, double qstep, double xmin,
@@ -84,6 +141,18 @@ __global__ __launch_bounds__(64 * kFbWaves) void k_fb_table(int which, const dou
 
 namespace gra_hip {
 
+hipError_t launch_density_pre(const ElasticAmp& A, int nf, double kmin, double kstep, double* pre,
+                              hipStream_t st) {
+  hipLaunchKernelGGL(k_density_pre, dim3((nf + 256) / 256), dim3(256), 0, st, A, nf, kmin, kstep,
+                     pre);
+  return hipGetLastError();
+}
+hipError_t launch_screening_pre(const double* mbt, int n_bt, double bmin, double bstep, int nf,
+                                double step, double* pre, hipStream_t st) {
+  hipLaunchKernelGGL(k_screening_pre, dim3((nf + 256) / 256), dim3(256), 0, st, mbt, n_bt, bmin,
+                     bstep, nf, step, pre);
+  return hipGetLastError();
+}
 hipError_t launch_fb_table(int which, const double* pre, int nf, double qmin, double qstep,
                            double xmin, double xstep, int nrows, double factor, double* out,
                            hipStream_t st, const double* xs) {

@@ -111,11 +111,9 @@ __device__ __forceinline__ double exp2_64(double x) {
   p = __builtin_fma(p, r, 1.0);
   return __builtin_ldexp(p, (int)n);
 }
-// cos and sin of 2 pi x: x less its nearest quarter, |theta| <= pi / 4, polynomials in
-// theta^2 through the Chebyshev nodes (relative errors 7e-18 and 1.3e-17)
-__device__ __forceinline__ void sincos_rev64(double x, double& sn, double& cs) {
-  const double q = __builtin_rint(4.0 * x);
-  const double th = __builtin_fma(-0.25, q, x) * 6.2831853071795865;
+// cos and sin of q pi / 2 + th, |th| <= pi / 4, q a whole number: polynomials in th^2
+// through the Chebyshev nodes (relative errors 7e-18 and 1.3e-17)
+__device__ __forceinline__ void sincos_quarter64(double q, double th, double& sn, double& cs) {
   const double z = th * th;
   double c = -1.1353379638297575e-11;
   c = __builtin_fma(c, z, 2.0875582380663952e-09);
@@ -136,6 +134,11 @@ __device__ __forceinline__ void sincos_rev64(double x, double& sn, double& cs) {
   const double a = (k & 1) ? s : c, b = (k & 1) ? c : s;
   cs = ((k + 1) & 2) ? -a : a;
   sn = (k & 2) ? -b : b;
+}
+// cos and sin of 2 pi x: x less its nearest quarter
+__device__ __forceinline__ void sincos_rev64(double x, double& sn, double& cs) {
+  const double q = __builtin_rint(4.0 * x);
+  sincos_quarter64(q, __builtin_fma(-0.25, q, x) * 6.2831853071795865, sn, cs);
 }
 
 // Record of a screened point for the folded nodes, written by k_tree

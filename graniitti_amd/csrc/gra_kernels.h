@@ -77,6 +77,15 @@ hipError_t launch_unweight(const double* w, uint64_t n, double wmax, uint64_t se
 // x_i = xs[i] when xs is given), out_i = factor * CSIntegral_q[pre_q J0(m(x_i) q_v) q_v],
 // q_v = qmin + q qstep, m(x) = x (density, which = 0) or sqrt(max(x, 0)) (screening,
 // which = 1).
+// Constants of the elastic amplitude of the density integrand
+struct ElasticAmp {
+  double s, gN, fc1, fc2, fc3, mpi, delta, slope;
+};
+// Factors of the density and the screening integrand at nf + 1 quadrature nodes (re, im)
+hipError_t launch_density_pre(const ElasticAmp& A, int nf, double kmin, double kstep, double* pre,
+                              hipStream_t st);
+hipError_t launch_screening_pre(const double* mbt, int n_bt, double bmin, double bstep, int nf,
+                                double step, double* pre, hipStream_t st);
 hipError_t launch_fb_table(int which, const double* pre, int nf, double qmin, double qstep,
                            double xmin, double xstep, int nrows, double factor, double* out,
                            hipStream_t st, const double* xs);
