@@ -684,9 +684,18 @@ int build_eikonal(gra_handle* h, const char* cache_dir) {
   const int NF = c.n_fb;
   DevBuf d_pre, d_out, d_mbt;
   const int nrow_max = std::max(std::max(c.n_bt, c.n_kt2) + 1, c.eik_log_nodes);
-  if (d_pre.ensure(sizeof(double) * 2 * (NF + 1)) || d_out.ensure(sizeof(double) * 2 * nrow_max))
+  if (d_pre.ensure(sizeof(double) * 2 * (NF + 1)) || d_out.ensure(sizeof(double) * 3 * nrow_max))
     return fail(h, GRA_E_NOMEM, "eikonal table buffers");
-  std::vector<double> out(2 * (size_t)nrow_max);
+  // The rows of the table kernel, rounded by it but for values that round through text
+  auto table_rows = [&](std::vector<double>& T, int n) -> int {
+    T.resize(3 * (size_t)n);
+    GRA_HIP_CHECK(h, hipMemcpyAsync(T.data(), d_out.p, sizeof(double) * T.size(),
+                                    hipMemcpyDeviceToHost, h->stream));
+    GRA_HIP_CHECK(h, hipStreamSynchronize(h->stream));
+    for (double& v : T)
+      if (!round15_exact(v)) v = round15_text(v);
+    return GRA_OK;
+  };
   // Density Omega(bt): pre_q = SingleAmpElastic(s, -kt_q^2)
   const double kmin = 1E-9, kmax = 30.0, kstep = (kmax - kmin) / NF;
   const double bmin = 1E-6, bmax = 10.0 / gev2fm(), bstep = (bmax - bmin) / c.n_bt;
@@ -697,16 +706,7 @@ int build_eikonal(gra_handle* h, const char* cache_dir) {
     GRA_HIP_CHECK(h, launch_fb_table(0, d_pre.as<double>(), NF, kmin, kstep, bmin, bstep,
                                      c.n_bt + 1, 1 / (2.0 * GRA_PI * P.s), d_out.as<double>(),
                                      h->stream, nullptr));
-    GRA_HIP_CHECK(h, hipMemcpyAsync(out.data(), d_out.p, sizeof(double) * 2 * (c.n_bt + 1),
-                                    hipMemcpyDeviceToHost, h->stream));
-    GRA_HIP_CHECK(h, hipStreamSynchronize(h->stream));
-    h->mbt.resize(3 * (size_t)(c.n_bt + 1));
-    for (int i = 0; i <= c.n_bt; ++i) {
-      h->mbt[3 * i] = round15(bmin + i * bstep);
-      h->mbt[3 * i + 1] = round15(out[2 * i]);
-      h->mbt[3 * i + 2] = round15(out[2 * i + 1]);
-    }
-    return GRA_OK;
+    return table_rows(h->mbt, c.n_bt + 1);
   });
   if (r != GRA_OK) return r;
   // Screening amplitude A_eik(kt^2): pre_q = i (1 - exp(i Omega(bt_q) / 2))
@@ -726,16 +726,7 @@ int build_eikonal(gra_handle* h, const char* cache_dir) {
     GRA_HIP_CHECK(h, launch_fb_table(1, d_pre.as<double>(), NF, bmin, STEP, amin, astep,
                                      c.n_kt2 + 1, (2.0 * P.s) * (2.0 * GRA_PI),
                                      d_out.as<double>(), h->stream, nullptr));
-    GRA_HIP_CHECK(h, hipMemcpyAsync(out.data(), d_out.p, sizeof(double) * 2 * (c.n_kt2 + 1),
-                                    hipMemcpyDeviceToHost, h->stream));
-    GRA_HIP_CHECK(h, hipStreamSynchronize(h->stream));
-    h->msa.resize(3 * (size_t)(c.n_kt2 + 1));
-    for (int i = 0; i <= c.n_kt2; ++i) {
-      h->msa[3 * i] = round15(amin + i * astep);
-      h->msa[3 * i + 1] = round15(out[2 * i]);
-      h->msa[3 * i + 2] = round15(out[2 * i + 1]);
-    }
-    return GRA_OK;
+    return table_rows(h->msa, c.n_kt2 + 1);
   });
   if (r != GRA_OK) return r;
   // A_eik at log-spaced kt nodes: the same Fourier-Bessel integral as the MSA

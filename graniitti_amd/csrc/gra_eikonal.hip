@@ -6,6 +6,7 @@
 #include "gra_device.h"
 #include "gra_fold.h"
 #include "gra_kernels.h"
+#include "gra_round15.h"
 
 namespace {
 
@@ -132,9 +133,14 @@ __global__ __launch_bounds__(64 * kFbWaves) void k_fb_table(int which, const dou
     sr += __shfl_xor(sr, o);
     si += __shfl_xor(si, o);
   }
-  if (lane != 0) return;
-  out[2 * i] = ((sr * qstep) / 3.0) * factor;
-  out[2 * i + 1] = ((si * qstep) / 3.0) * factor;
+  const double re = ((sr * qstep) / 3.0) * factor, im = ((si * qstep) / 3.0) * factor;
+  if (xs) {
+    if (lane < 2) out[2 * i + lane] = lane ? im : re;
+  } else if (lane < 3) {
+    // a table row (x, re, im); values that need the text round trip stay as they are
+    const double v = lane == 0 ? xv : lane == 1 ? re : im;
+    out[3 * i + lane] = gra_hip::round15_exact(v) ? gra_hip::round15_arith(v) : v;
+  }
 }
 
 }  // namespace

@@ -73,8 +73,9 @@ hipError_t launch_accept(const double* W, const double* vw, const uint8_t* flags
 hipError_t launch_unweight(const double* w, uint64_t n, double wmax, uint64_t seed, uint8_t* acc,
                            unsigned long long* counts, hipStream_t st);
 
-// Eikonal Fourier-Bessel tables: rows i = 0..nrows-1 at x_i = xmin + i xstep (or
-// x_i = xs[i] when xs is given), out_i = factor * CSIntegral_q[pre_q J0(m(x_i) q_v) q_v],
+// Eikonal Fourier-Bessel tables: rows i = 0..nrows-1 (x_i, re_i, im_i) at x_i = xmin + i
+// xstep, rounded to 15 digits where round15_exact holds, or, when xs is given, (re_i, im_i)
+// at x_i = xs[i], not rounded; re_i + i im_i = factor * CSIntegral_q[pre_q J0(m(x_i) q_v) q_v],
 // q_v = qmin + q qstep, m(x) = x (density, which = 0) or sqrt(max(x, 0)) (screening,
 // which = 1).
 // Constants of the elastic amplitude of the density integrand
