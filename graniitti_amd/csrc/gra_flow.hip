@@ -1176,17 +1176,32 @@ __global__ void k_adam(float* __restrict__ th, const float* __restrict__ g, floa
   th[i] -= lr * (mi * c1) / (sqrtf(vi * c2) + eps);
 }
 
+// The weights that one launch of k_weights_bf16 copies, a block row each: their offsets in
+// the parameters and in the copies, and their columns
+constexpr int kWeightSlots = 64;
+struct WeightSlots {
+  size_t from[kWeightSlots], to[kWeightSlots];
+  int N[kWeightSlots];
+};
 // W[Kin x N] (row-major, fp32) -> Wt16[N x Kin], W16[Kin x N] and, in the order in which
 // the lanes of the fused layer's MFMAs hold it, Wf16 (bf16): 1 KB blocks of 16 columns by
 // 32 rows, in a block lane l's eight values, rows 8 (l / 16) .. of column l % 16. N and Kin
 // are multiples of 64. A block is one contiguous load of a wave; out of Wt16 it was 16
 // half cache lines, and a product's lines (49 KB for three tiles of eight waves) did not
-// stay in the 32 KB L1 until the next load took their other halves.
-__global__ void k_weights_bf16(const float* __restrict__ W, int Kin, int N, __bf16* __restrict__ Wt16,
-                               __bf16* __restrict__ W16, __bf16* __restrict__ Wf16,
-                               float* __restrict__ Wt32) {
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
+// stay in the 32 KB L1 until the next load took their other halves. A launch takes up to 64
+// weights: twelve launches of 4.6 us
+// a step are one of 4 (6 layers of 2 x 128).
+__global__ void k_weights_bf16(const float* __restrict__ theta, WeightSlots S, int Kin,
+                               __bf16* __restrict__ Wt16, __bf16* __restrict__ W16,
+                               __bf16* __restrict__ Wf16, float* __restrict__ Wt32) {
+  const int idx = blockIdx.x * blockDim.x + threadIdx.x, N = S.N[blockIdx.y];
   if (idx >= Kin * N) return;
+  const float* W = theta + S.from[blockIdx.y];
+  const size_t to = S.to[blockIdx.y];
+  Wt16 += to;
+  W16 += to;
+  Wf16 += to;
+  Wt32 += to;
   const int k = idx / N, c = idx % N;
   const float w = W[idx];
   Wt16[(size_t)c * Kin + k] = (__bf16)w;
@@ -1818,20 +1833,22 @@ static float* act32_of(FlowState* F, int l, int i) {
 
 // bf16 / fp32 copies of the GEMM weights (hidden layers and output) of every layer
 static int refresh_weights(gra_handle* h, FlowState* F) {
-  int slot = 0;
-  for (int l = 0; l < F->L; ++l) {
-    const FlowLayerHost& Ly = F->layers[l];
-    for (int i = 1; i <= F->depth; ++i) {
-      const bool out = (i == F->depth);
-      const size_t off = out ? Ly.oWo : Ly.oWh[i];
-      const int N = out ? F->ldp : F->H;
-      const int n = F->H * N;
-      hipLaunchKernelGGL(k_weights_bf16, dim3((n + 255) / 256), dim3(256), 0, h->stream,
-                         F->theta.as<float>() + off, F->H, N, F->wt16.as<__bf16>() + F->wofs[slot],
-                         F->w16.as<__bf16>() + F->wofs[slot], F->wf16.as<__bf16>() + F->wofs[slot],
-                         F->wt32.as<float>() + F->wofs[slot]);
-      ++slot;
+  const int n = F->L * F->depth;
+  for (int s0 = 0; s0 < n; s0 += kWeightSlots) {
+    const int ns = std::min(kWeightSlots, n - s0);
+    WeightSlots S;
+    std::memset(&S, 0, sizeof(S));
+    for (int k = 0; k < ns; ++k) {
+      const FlowLayerHost& Ly = F->layers[(s0 + k) / F->depth];
+      const int i = 1 + (s0 + k) % F->depth;
+      S.from[k] = i == F->depth ? Ly.oWo : Ly.oWh[i];
+      S.to[k] = F->wofs[s0 + k];
+      S.N[k] = i == F->depth ? F->ldp : F->H;
     }
+    const int most = F->H * std::max(F->ldp, F->H);
+    hipLaunchKernelGGL(k_weights_bf16, dim3((most + 255) / 256, ns), dim3(256), 0, h->stream,
+                       F->theta.as<float>(), S, F->H, F->wt16.as<__bf16>(), F->w16.as<__bf16>(),
+                       F->wf16.as<__bf16>(), F->wt32.as<float>());
   }
   GRA_HIP_CHECK(h, hipGetLastError());
   return GRA_OK;
