@@ -1190,7 +1190,7 @@ struct WeightSlots {
 // half cache lines, and a product's lines (49 KB for three tiles of eight waves) did not
 // stay in the 32 KB L1 until the next load took their other halves. A launch takes up to 64
 // weights: twelve launches of 4.6 us
-// a step are one of 4 (6 layers of 2 x 128).
+// a step are one of 8 (6 layers of 2 x 128).
 __global__ void k_weights_bf16(const float* __restrict__ theta, WeightSlots S, int Kin,
                                __bf16* __restrict__ Wt16, __bf16* __restrict__ W16,
                                __bf16* __restrict__ Wf16, float* __restrict__ Wt32) {
