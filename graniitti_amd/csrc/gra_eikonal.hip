@@ -49,6 +49,12 @@ __device__ __forceinline__ double bessj0(double X) {
 // loops (pow, log, exp and sincos at 10001 nodes each) took 0.7 of 3.4 ms of a set-up, here
 // 9 us.
 //
+// Each is multiplied by its node and by its weight 1, 2 or 4 in the composite Simpson sum
+// (CSIntegral: h (f0 + 2 I_even + 4 I_odd + fN) / 3, include/Graniitti/MMath.h:378-394).
+__device__ __forceinline__ double simpson_node(int q, int nf, double v) {
+  return (q == 0 || q == nf) ? v : (q & 1) ? 4.0 * v : 2.0 * v;
+}
+
 // Density: pre_q = MEikonal::SingleAmpElastic(s, -kt_q^2), src/MEikonal.cc:139-154, with
 // form::S3HPL, S3PomAlpha and ReggeEta (src/MForm.cc:382-426)
 __global__ void k_density_pre(ElasticAmp A, int nf, double kmin, double kstep,
@@ -69,8 +75,9 @@ __global__ void k_density_pre(ElasticAmp A, int nf, double kmin, double kstep,
   double sn, cs;
   sincos(GRA_PI * alpha, &sn, &cs);
   const double a = ((A.gN * A.gN) * F) * F * pow(A.s, alpha);
-  pre[2 * q] = -((1.0 + cs) / sn) * a;  // eta = -(1 + exp(-i pi alpha)) / sin(pi alpha)
-  pre[2 * q + 1] = (sn / sn) * a;
+  const double w = simpson_node(q, nf, kt);
+  pre[2 * q] = -((1.0 + cs) / sn) * a * w;  // eta = -(1 + exp(-i pi alpha)) / sin(pi alpha)
+  pre[2 * q + 1] = (sn / sn) * a * w;
 }
 // Screening: pre_q = i (1 - exp(i Omega(bt_q) / 2)), Omega between the density table's rows
 // (x, re, im) as IArray1D::Interpolate1D takes it (src/MEikonal.cc:489-512)
@@ -78,6 +85,7 @@ __global__ void k_screening_pre(const double* __restrict__ T, int n_bt, double b
                                 int nf, double step, double* __restrict__ pre) {
   const int q = blockIdx.x * blockDim.x + threadIdx.x;
   if (q > nf) return;
+  const double w = simpson_node(q, nf, bmin + q * step);
   double b = bmin + q * step;
   if (b < bmin) b = bmin;
   int i = (int)floor((b - bmin) / bstep);
@@ -88,58 +96,63 @@ __global__ void k_screening_pre(const double* __restrict__ T, int n_bt, double b
   const double e = exp(-im / 2.0);
   double sn, cs;
   sincos(re / 2.0, &sn, &cs);
-  pre[2 * q] = e * sn;  // i (1 - e (cos + i sin))
-  pre[2 * q + 1] = 1.0 - e * cs;
+  pre[2 * q] = e * sn * w;  // i (1 - e (cos + i sin))
+  pre[2 * q + 1] = (1.0 - e * cs) * w;
 }
 
-// One wave per table row: lane l takes the quadrature nodes l, l + 64, ... (coalesced
+// Two table rows per wave: lane l takes the quadrature nodes l, l + 64, ... (coalesced
 // loads, and the same Bessel branch across the wave but at one boundary), whose parity is
 // the lane's, and a butterfly adds the lanes' sums in a fixed order. With one thread per
 // row 10001 rows were 40 blocks, each a serial chain of 10001 terms: 6.0 ms a table at 16%
 // of the CUs. As waves they fill the chip, bound by the FP64 VALU: 0.52 ms with a division,
-// a library root and sincos a term (207 instructions), 0.33 with bessj0's (150). Against
+// a library root and sincos a term (207 instructions), 0.33 with bessj0's (150), 0.29 with
+// the nodes' weights in pre and its loads shared by two rows (a set-up 1.35 -> 1.27 ms). Against
 // 80-bit sums of the same fit the tables are off by 3e-15 of their largest value, as before
 // or less (screening 5.2e-15 and 2.9e-15 at 3.5 and 6.5 TeV beams, now 3.1e-15, 0.9e-15).
-constexpr int kFbWaves = 4;  // rows per block
-__global__ __launch_bounds__(64 * kFbWaves) void k_fb_table(int which, const double* __restrict__ pre, int nf,
+constexpr int kFbWaves = 4;  // of two rows each, per block
+__global__ __launch_bounds__(64 * kFbWaves) void k_fb_table(int which, const double2* __restrict__ pre, int nf,
                                                   double qmin, double qstep, double xmin,
                                                   double xstep, int nrows, double factor,
                                                   const double* __restrict__ xs,
                                                   double* __restrict__ out) {
-  const int i = blockIdx.x * kFbWaves + (threadIdx.x >> 6);  // wave-uniform
+  const int i0 = 2 * (blockIdx.x * kFbWaves + (threadIdx.x >> 6));  // wave-uniform
   const int lane = threadIdx.x & 63;
-  if (i >= nrows) return;
-  const double xv = xs ? xs[i] : xmin + i * xstep;
-  const double m = (which == 0) ? xv : msq(xv);
-  double fr = 0.0, fi = 0.0;  // this lane's interior nodes
-  double er = 0.0, ei = 0.0;  // the end nodes f0 + fN (lanes 0 and nf mod 64)
+  if (i0 >= nrows) return;
+  double m[2], sr[2] = {0.0, 0.0}, si[2] = {0.0, 0.0};
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const int i = min(i0 + k, nrows - 1);  // an odd last row twice
+    const double xv = xs ? xs[i] : xmin + i * xstep;
+    m[k] = (which == 0) ? xv : msq(xv);
+  }
   for (int q = lane; q <= nf; q += 64) {
     const double qv = qmin + q * qstep;
-    const double j0 = bessj0(m * qv);
-    const double tr = (pre[2 * q] * j0) * qv, ti = (pre[2 * q + 1] * j0) * qv;
-    if (q == 0 || q == nf) {
-      er += tr;
-      ei += ti;
-    } else {
-      fr += tr;
-      fi += ti;
+    const double2 p = pre[q];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const double j0 = bessj0(m[k] * qv);
+      sr[k] = __builtin_fma(p.x, j0, sr[k]);
+      si[k] = __builtin_fma(p.y, j0, si[k]);
     }
   }
-  // CSIntegral: h (f0 + 2 I_even + 4 I_odd + fN) / 3, include/Graniitti/MMath.h:378-394
-  const double w = (lane & 1) ? 4.0 : 2.0;
-  double sr = er + w * fr, si = ei + w * fi;
 #pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    sr += __shfl_xor(sr, o);
-    si += __shfl_xor(si, o);
-  }
-  const double re = ((sr * qstep) / 3.0) * factor, im = ((si * qstep) / 3.0) * factor;
+  for (int o = 1; o < 64; o <<= 1)
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      sr[k] += __shfl_xor(sr[k], o);
+      si[k] += __shfl_xor(si[k], o);
+    }
+  // lanes 0 .. 2 and 32 .. 34 write a row each
+  const int k = lane >> 5, i = i0 + k, c = lane & 31;
+  if (i >= nrows) return;
+  const double re = (((k ? sr[1] : sr[0]) * qstep) / 3.0) * factor;
+  const double im = (((k ? si[1] : si[0]) * qstep) / 3.0) * factor;
   if (xs) {
-    if (lane < 2) out[2 * i + lane] = lane ? im : re;
-  } else if (lane < 3) {
+    if (c < 2) out[2 * i + c] = c ? im : re;
+  } else if (c < 3) {
     // a table row (x, re, im); values that need the text round trip stay as they are
-    const double v = lane == 0 ? xv : lane == 1 ? re : im;
-    out[3 * i + lane] = gra_hip::round15_exact(v) ? gra_hip::round15_arith(v) : v;
+    const double v = c == 0 ? xmin + i * xstep : c == 1 ? re : im;
+    out[3 * i + c] = gra_hip::round15_exact(v) ? gra_hip::round15_arith(v) : v;
   }
 }
 
@@ -162,8 +175,9 @@ hipError_t launch_screening_pre(const double* mbt, int n_bt, double bmin, double
 hipError_t launch_fb_table(int which, const double* pre, int nf, double qmin, double qstep,
                            double xmin, double xstep, int nrows, double factor, double* out,
                            hipStream_t st, const double* xs) {
-  hipLaunchKernelGGL(k_fb_table, dim3((nrows + kFbWaves - 1) / kFbWaves), dim3(64 * kFbWaves), 0, st,
-                     which, pre, nf, qmin, qstep, xmin, xstep, nrows, factor, xs, out);
+  const int per = 2 * kFbWaves;
+  hipLaunchKernelGGL(k_fb_table, dim3((nrows + per - 1) / per), dim3(64 * kFbWaves), 0, st, which,
+                     (const double2*)pre, nf, qmin, qstep, xmin, xstep, nrows, factor, xs, out);
   return hipGetLastError();
 }
 

@@ -75,14 +75,15 @@ hipError_t launch_unweight(const double* w, uint64_t n, double wmax, uint64_t se
 
 // Eikonal Fourier-Bessel tables: rows i = 0..nrows-1 (x_i, re_i, im_i) at x_i = xmin + i
 // xstep, rounded to 15 digits where round15_exact holds, or, when xs is given, (re_i, im_i)
-// at x_i = xs[i], not rounded; re_i + i im_i = factor * CSIntegral_q[pre_q J0(m(x_i) q_v) q_v],
+// at x_i = xs[i], not rounded; re_i + i im_i = factor * qstep / 3 * sum_q pre_q J0(m(x_i) q_v),
 // q_v = qmin + q qstep, m(x) = x (density, which = 0) or sqrt(max(x, 0)) (screening,
 // which = 1).
 // Constants of the elastic amplitude of the density integrand
 struct ElasticAmp {
   double s, gN, fc1, fc2, fc3, mpi, delta, slope;
 };
-// Factors of the density and the screening integrand at nf + 1 quadrature nodes (re, im)
+// Factors of the density and the screening integrand at nf + 1 quadrature nodes (re, im),
+// times the node and its weight in the composite Simpson sum
 hipError_t launch_density_pre(const ElasticAmp& A, int nf, double kmin, double kstep, double* pre,
                               hipStream_t st);
 hipError_t launch_screening_pre(const double* mbt, int n_bt, double bmin, double bstep, int nf,
