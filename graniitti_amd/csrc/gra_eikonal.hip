@@ -107,8 +107,9 @@ __global__ void k_screening_pre(const double* __restrict__ T, int n_bt, double b
 // of the CUs. As waves they fill the chip, bound by the FP64 VALU: 0.52 ms with a division,
 // a library root and sincos a term (207 instructions), 0.33 with bessj0's (150), 0.29 with
 // the nodes' weights in pre and its loads shared by two rows (a set-up 1.35 -> 1.27 ms). Against
-// 80-bit sums of the same fit the tables are off by 3e-15 of their largest value, as before
-// or less (screening 5.2e-15 and 2.9e-15 at 3.5 and 6.5 TeV beams, now 3.1e-15, 0.9e-15).
+// 80-bit sums of the same fit the tables are off, relative to their largest value and for
+// beams of 3.5 and 6.5 TeV, by 3.1e-15 and 2.9e-15 (density; 2.7e-15 and 3.6e-15 with the
+// library functions) and 3.1e-15 and 0.9e-15 (screening; 5.2e-15 and 2.9e-15).
 constexpr int kFbWaves = 4;  // of two rows each, per block
 __global__ __launch_bounds__(64 * kFbWaves) void k_fb_table(int which, const double2* __restrict__ pre, int nf,
                                                   double qmin, double qstep, double xmin,
