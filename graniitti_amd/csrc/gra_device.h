@@ -38,10 +38,13 @@ __device__ __forceinline__ dv4 v4scale(dv4 a, double d) {
 }
 // sqrt(x), 0 for x <= 0 and NaN, rounded as sqrt rounds it: Goldschmidt's iteration from
 // the hardware's seed and two residual corrections, without the scaling that sqrt needs
-// for x below 2^-767 (here a value below 1e-150 comes out for x below 1e-300). It has six
+// for x below 2^-767 (here a value below 1e-150 comes out for x below 1e-300). It has five
 // instructions less of 17; a node of the tensor pair takes ten roots, a tree point some 40:
 // 2^18 screened rho rho points 4.04 -> 3.98 ms, 2^20 unscreened points 267 -> 263 us. Equal
-// to sqrt in 3e10 values of 2^-900 .. 2^900, squares and midpoints among them.
+// to sqrt in 3e10 values of 2^-900 .. 2^900, squares and midpoints among them. For x = Inf
+// the iteration is Inf 0 = NaN, which guards of the form E > bound would let through: the
+// last step, the fixup of a division s / 1, puts Inf in its place (no time of its own in
+// either of the two launches).
 __device__ __forceinline__ double msq(double x) {
 #pragma clang fp contract(off)
   const double s = x > 0.0 ? x : 0.0;
@@ -51,7 +54,8 @@ __device__ __forceinline__ double msq(double x) {
   g = __builtin_fma(g, r, g);
   h = __builtin_fma(h, r, h);
   g = __builtin_fma(__builtin_fma(-g, g, s), h, g);
-  return __builtin_fma(__builtin_fma(-g, g, s), h, g);
+  g = __builtin_fma(__builtin_fma(-g, g, s), h, g);
+  return __builtin_amdgcn_div_fixup(g, 1.0, s);  // Inf for s = Inf, else g
 }
 __device__ __forceinline__ double p3mod2(dv4 a) { return a.x * a.x + a.y * a.y + a.z * a.z; }
 __device__ __forceinline__ double m2of(dv4 a) { return a.e * a.e - p3mod2(a); }
