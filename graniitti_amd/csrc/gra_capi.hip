@@ -1315,10 +1315,17 @@ extern "C" int gra_hip_vegas_iterate(gra_handle* h, const gra_grid* grid, uint64
   if (h->d_part_hist.ensure(sizeof(double) * H * nblk) ||
       h->d_part_scal.ensure(sizeof(double) * kIterScalars * nblk))
     return fail(h, GRA_E_NOMEM, "VEGAS buffers");
-  // the reduction leaves the statistics in pinned memory, without a copy
-  if (!pin_ensure(h, sizeof(double) * (kIterScalars + H)))
-    return fail(h, GRA_E_NOMEM, "pinned VEGAS statistics");
-  const double* s = (double*)h->h_pin;
+  // the reduction leaves the statistics in pinned memory, without a copy; where there is
+  // none to be had, in a device buffer
+  const size_t stats = sizeof(double) * (kIterScalars + H);
+  const bool pinned = pin_ensure(h, stats);
+  std::vector<double> own;
+  if (!pinned) {
+    own.resize(kIterScalars + H);
+    if (h->d_x.ensure(stats)) return fail(h, GRA_E_NOMEM, "VEGAS statistics");
+  }
+  double* d_stats = pinned ? (double*)h->h_pin : h->d_x.as<double>();
+  const double* s = pinned ? (const double*)h->h_pin : own.data();
   r = upload_grid(h, grid);
   if (r) return r;
   r = run_integrand(h, h->d_grid.as<double>(), (unsigned int)grid->bins, seed, iter, 0, nullptr,
@@ -1329,9 +1336,10 @@ extern "C" int gra_hip_vegas_iterate(gra_handle* h, const gra_grid* grid, uint64
   GRA_HIP_CHECK(h, launch_accumulate(h->d_W.as<double>(), h->d_vw.as<double>(),
                                      h->d_bins.as<uint8_t>(), h->d_flags.as<uint8_t>(), n_calls, D,
                                      nblk, h->d_part_hist.as<double>(),
-                                     h->d_part_scal.as<double>(), (double*)h->h_pin,
-                                     h->stream));
+                                     h->d_part_scal.as<double>(), d_stats, h->stream));
   time_end(h, TS_ACCUM);
+  if (!pinned)
+    GRA_HIP_CHECK(h, hipMemcpyAsync(own.data(), d_stats, stats, hipMemcpyDeviceToHost, h->stream));
   GRA_HIP_CHECK(h, hipStreamSynchronize(h->stream));
   time_collect(h, true, h->P.screening != 0, true);
   std::memset(out, 0, sizeof(*out));
