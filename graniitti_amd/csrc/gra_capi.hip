@@ -990,7 +990,7 @@ int run_integrand(gra_handle* h, const double* d_grid, unsigned int bins, uint64
 // object, so that gra_hip_eval_points_noalloc calls no allocator. Its device
 // address comes from hipGetSymbolAddress once per device, at the first handle
 // creation on that device; host code uses that address, never the symbol.
-// Layout: [0, 256) the candidate counter, then the candidate records, the VEGAS
+// Layout: [0, 256) the two candidate counters, then the candidate records, the VEGAS
 // weights (unused here: the points come from the caller) and the bin bytes, each
 // 256-byte aligned.
 // ---------------------------------------------------------------------------
@@ -1003,7 +1003,7 @@ void* g_scratch_ptr[kMaxDevices] = {};
 
 inline size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
-// Bytes of scratch n points of this process need (counter, records, weights, bins)
+// Bytes of scratch n points of this process need (counters, records, weights, bins)
 size_t noalloc_bytes(const gra_handle* h, uint64_t n) {
   const size_t recb = f32_kernels(h->P) ? k32::loop_record_bytes(h->P)
                                         : k64::loop_record_bytes(h->P);

@@ -77,7 +77,7 @@ __global__ void k_density_pre(ElasticAmp A, int nf, double kmin, double kstep,
   const double a = ((A.gN * A.gN) * F) * F * pow(A.s, alpha);
   const double w = simpson_node(q, nf, kt);
   pre[2 * q] = -((1.0 + cs) / sn) * a * w;  // eta = -(1 + exp(-i pi alpha)) / sin(pi alpha)
-  pre[2 * q + 1] = (sn / sn) * a * w;
+  pre[2 * q + 1] = (sn / sn) * a * w;  // the factor is 1, or NaN at a pole of eta
 }
 // Screening: pre_q = i (1 - exp(i Omega(bt_q) / 2)), Omega between the density table's rows
 // (x, re, im) as IArray1D::Interpolate1D takes it (src/MEikonal.cc:489-512)
